@@ -67,7 +67,15 @@ namespace cvsa {
 // A q-head's o is D / 4 float4 chunks.
 __host__ __device__ constexpr int part_stride(int D) { return D + 4; }
 constexpr int kMaxSplits = 256;            // partials per head (and workgroups per launch)
+// Waves per workgroup, one per SIMD.  Eight waves (two per SIMD, the same
+// tiles in flight per wave) measured slower: the listed decode 17.3 against
+// 17.1 us at cfg3 and 44.4 against 43.2 us at B = 32 (ragged 8K contexts),
+// dense at B = 4, 64K 186 against 178 us.
+constexpr int kWavesPerWg = 4;
 constexpr int kMinPagesPerWave = 2;        // pages per wave of a split, at least
+// Waves per SIMD the listed kernels' registers are held to: launches of more
+// than one workgroup per CU overlap one's hand-off with another's walk.
+constexpr int walk_waves(int D) { return D > 128 ? 2 : 4; }
 
 struct DecodeArgs {
   const uint16_t *q;
@@ -282,7 +290,7 @@ constexpr int kMaxHeads = 4096;  // B * H_kv of one launch
 constexpr int kMergeGroup = 16;
 constexpr int kTwoLevelMin = 48;
 constexpr int kGroupCounters = 2 * 256;  // 2 x the largest stream-K grid
-constexpr int kMinPagesPerWg = kMinPagesPerWave * 4;
+constexpr int kMinPagesPerWg = kMinPagesPerWave * kWavesPerWg;
 
 struct Partition {
   int T, n, q, r;  // pages, workgroups, T / n, T % n
@@ -317,6 +325,7 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 struct PartBuf {
   static constexpr int kCpolAgent = 16;         // sc1
   static constexpr int kRsrcWord3 = 0x00020000;  // 32-bit data format, raw
+  static constexpr uint32_t kNoRow = 0x3ffffffcu;  // past any launch's partials (< 2 GiB)
   __amdgpu_buffer_rsrc_t r;
   __device__ __forceinline__ PartBuf(float *base, uint32_t bytes)
       : r(__builtin_amdgcn_make_buffer_rsrc(base, (short)0, (int)bytes, kRsrcWord3)) {}
@@ -381,26 +390,26 @@ struct MergeLds {
   f32x4 acc[NT];
 };
 
-// o chunks of one merging thread requested together (KB of merge_partials):
-// 16 in the listed decode, whose merge ends the kernel, so a cfg3-sized head
-// (32 splits) is read in one memory round trip; 8 in the stream-K kernel,
-// whose merge sits inside its segment loop, where 16 would cost it an
-// occupancy step.
-constexpr int kMergeBatchListed = 16;
-constexpr int kMergeBatchStreamK = 8;
+// o chunks of one merging thread requested together: as many as read a
+// 32-split head (cfg3's) in one memory round trip over the J threads that
+// share a chunk, 4 to 16 of them (8 in the stream-K kernel, whose merge sits
+// inside its segment loop, where 16 would spill).
+constexpr int merge_batch(int J, int most) {
+  return J >= 8 ? 4 : 32 / J < most ? 32 / J : most;
+}
 
 // Merge of a head's n_act split partials by the last of its workgroups
 // (partial sp at row offset head_off + sp * row_step rows).  TO_PART: the
 // merged (o, m, l) of the rows go to the partial row at part_off instead of
 // the outputs (the first level of a two-level merge; no counters booked).
 // Thread t owns float4 chunk c = t % NC of the head's G x D outputs and the
-// splits j, j + J, ... (j = t / NC); their o chunks are loaded KB at a time,
-// the first KB together with the (m, l) pairs.  When the
+// splits j, j + J, ... (j = t / NC); their o chunks are loaded KB = merge_batch at a
+// time, the first KB together with the (m, l) pairs.  When the
 // outputs hold more chunks than the workgroup has threads (G x D > 4 NT) each
 // thread takes chunks t, t + NT, ... in turn, every split of each.  The
 // (m, l) pairs go to LDS first; one wave per q-head turns them into the
 // weights exp(m_sp - M) and the totals (M, L).
-template <int G, int D, int NT, int KB, bool TO_PART = false>
+template <int G, int D, int NT, int KMAX, bool TO_PART = false>
 __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBuf &pb,
                                                uint32_t head_off, int n_act, int bh, int n,
                                                int nv, MergeLds<G, NT> &s, int row_step = 1,
@@ -412,6 +421,7 @@ __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBu
   constexpr int J = NT / NC > 0 ? NT / NC : 1;
   constexpr int NPASS = (NC + NT - 1) / NT;
   constexpr int NW = NT / kWave;
+  constexpr int KB = merge_batch(J, KMAX);
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = t >> 6;
@@ -424,8 +434,10 @@ __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBu
   auto load_batch = [&](int g, int d0, int b0, f32x4 (&v)[KB]) {
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
-      const int sp = min(j + (b0 + k) * J, n_act - 1);
-      v[k] = pb.load4(head_off + (uint32_t)sp * row_elems + g * kPartStride + d0);
+      // Past the thread's splits: out of the buffer's range, not read.
+      const uint32_t off = head_off + (uint32_t)(j + (b0 + k) * J) * row_elems +
+                           g * kPartStride + d0;
+      v[k] = pb.load4(b0 + k < per_lane ? off : PartBuf::kNoRow);
     }
   };
   f32x4 cur[KB];
@@ -496,30 +508,55 @@ __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBu
 
 // ---------------------------------------------------------------- engines
 // A page engine owns one wave's softmax state for the G query heads of a KV
-// head and applies pages to it.  Page = the K and V rows of one page held in
-// registers (fetched PD pages ahead); consume() applies one page; finish()
-// leaves the wave's (o, m, l) in LDS.
+// head and applies tiles to it.  One tile's K rows (kr) and V rows (vr) are
+// in registers at a time: each is staged to LDS as soon as it arrives and the
+// next tile's loads are issued into the same registers at once, so a wave
+// always has about one tile in flight; finish() leaves the wave's (o, m, l)
+// in LDS.
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-// MFMA engine: the G query heads (padded to 16) of a KV head against a page
-// of 16 tokens are two small dense tiles for the matrix cores.
+// RNE bf16 pair (v_cvt_pk_bf16_f32): the bits of f32_to_bf16_bits.
+__device__ __forceinline__ uint32_t cvt_bf16x2(float lo, float hi) {
+  const f32x2 x = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
+}
+
+// No tile: ctx - (kNoTile << 4) < 0, so it has no valid token, and its loads
+// are dropped.
+constexpr int kNoTile = 1 << 26;
+
+// MFMA engine: the G query heads (padded to 16) of a KV head against a tile
+// of 16 tokens are two small dense products for the matrix cores.
 //   S = K Q^T: v_mfma_f32_16x16x32_bf16, four d-chunks of 32.  A operand =
-//     K rows (lane l: token l%16, d 32kk + 8(l/16) .. +8, one 16-byte load),
-//     B operand = Q^T (loaded once), result lane l: head l%16, tokens
-//     4(l/16) .. +4.
-//   O += P V: v_mfma_f32_16x16x16_bf16, eight 16-column blocks of d.  The S
-//     result layout is exactly the A operand layout of P (head l%16, tokens
-//     4(l/16) .. +4), so P needs no data movement; it is split into a bf16
-//     high part and a bf16 remainder (two MFMAs) to keep ~16 mantissa bits.
-//     The B operand wants 4 tokens of one d column per lane: the V page goes
-//     through a wave-private LDS tile (rows padded to 272 bytes so the four
-//     lane groups read disjoint banks).  Result lane l: heads 4(l/16) .. +4,
-//     d column 16 blk + l%16.
+//     K rows (lane l: token l%16, d 32kk + 8(l/16) .. +8), B operand = Q^T
+//     (loaded once), result lane l: head l%16, tokens 4(l/16) .. +4.
+//   O += P V: P is split into a bf16 high part and a bf16 remainder to keep
+//     ~16 mantissa bits; lane l holds both for head l%16, tokens 4(l/16) ..
+//     +4 (the S result layout), which are the eight A operands of one
+//     v_mfma_f32_16x16x32_bf16 against the tile's V columns taken twice, one
+//     MFMA per 16 columns of d.  The B operand wants 4 tokens of one d column
+//     per lane: ds_read_b64_tr_b16 transposes it out of the row-major V tile.
+//     Result lane l: heads 4(l/16) .. +4, d column 16 blk + l%16.
 // Softmax state: m and the running l of head l%16 live in the four lanes of
 // that head; a rescale of O rows goes through LDS (16 factors per wave).
+//
+// What bounds the walk is HBM reads of 256-byte rows 2 KiB apart.  K and V
+// rows are both read whole (LPR lanes of 16 bytes per row, nontemporal) and
+// K reaches the A operand layout through LDS: reading K in that layout
+// directly (64 bytes of each of 16 rows per instruction, every line requested
+// twice) streams 5% slower, and so do two tiles in flight per wave instead of
+// one (a gather of the cfg3 selection, 64 MiB, without compute: 13.8 us with
+// two tiles in flight, 12.8 with one, 12.15 with whole K rows as well; of
+// B = 32, 128 pages per head, 256 MiB: 47.6, 46.5 and 43.6 us).  Tiles past
+// the end of a walk are not read: their loads go out of the tile's buffer
+// range and are dropped there (prefetches that read a wave's last tile again
+// instead cost the cfg3 listed decode a quarter more requests).  With the
+// engine of two tiles in flight the kernels took: listed 19.1 -> 17.1 us at
+// cfg3, 47.2 -> 43.2 us at B = 32 (ragged 8K), 10.3 -> 9.0 us at B = 1, 8K;
+// dense at B = 4, 64K, G = 8 185-191 -> 178 us.
 template <int G, int D, int TS>
 struct MfmaEngine {
   static_assert(G <= 16, "GQA group larger than the MFMA tile");
@@ -533,37 +570,43 @@ struct MfmaEngine {
   static __device__ __forceinline__ int tlog(const DecodeArgs &a) { return TS >= 0 ? 4 : a.tl; }
   static constexpr int NK = D / 32;         // S = K Q^T MFMAs (32 dimensions each)
   static constexpr int NB = D / 16;         // O column blocks (16 dimensions each)
-  static constexpr int LPR = D / 8;         // lanes per V row (16 bytes each)
-  static constexpr int RPL = kWave / LPR;   // V rows per wave load
-  static constexpr int NV = kPageTokens / RPL;  // V loads per page
-  static constexpr int kVRow = D + 8;       // LDS row of the V tile, in bf16
-  struct Page {
-    uint4 k[NK], v[NV];
+  static constexpr int LPR = D / 8;         // lanes per K or V row (16 bytes each)
+  static constexpr int RPL = kWave / LPR;   // rows per wave load
+  static constexpr int NL = kPageTokens / RPL;  // K (or V) loads per tile
+  static constexpr int kRow = D + 8;        // LDS row of a K or V tile, in bf16
+  struct Tiles {
+    uint16_t k[kPageTokens * kRow], v[kPageTokens * kRow];
   };
+  // One wave's LDS: the tiles of the walk, then the wave's o.
   struct Lds {
-    uint16_t v[kPageTokens * kVRow];
+    union {
+      Tiles t;
+      float o[G * D];
+    };
     float alpha[16];
   };
+  static_assert(sizeof(float) * G * D <= sizeof(Tiles), "a wave's o fits its tiles");
 
   float4_t o[NB];
   bf16x8_t qb[NK];
+  uint4 kr[NL], vr[NL];  // the tile in flight
   float m_g, l_g;
   int lane;
   int rmask;  // rows of a tile - 1: a load of row r reads row r & rmask
-  int64_t koff, voff, row_stride;
+  uint32_t voff, row_bytes, tile_bytes;
   float scale;
 
-  __device__ __forceinline__ void init(const DecodeArgs &a, int b, int h, int lane_, Lds &) {
+  __device__ __forceinline__ void init(const DecodeArgs &a, int b, int h, int lane_) {
     lane = lane_;
     scale = a.scale;
     rmask = (1 << tlog(a)) - 1;
-    row_stride = (int64_t)a.H_kv * D;
+    row_bytes = (uint32_t)(a.H_kv * D * 2);
+    tile_bytes = row_bytes << tlog(a);
     const int c16 = lane & 15, grp = lane >> 4;
-    koff = (int64_t)h * D + (c16 & rmask) * row_stride + 8 * grp;
-    voff = (int64_t)h * D + ((lane / LPR) & rmask) * row_stride + 8 * (lane % LPR);
+    voff = ((lane / LPR) & rmask) * row_bytes + (uint32_t)(h * D + 8 * (lane % LPR)) * 2;
     // Rows past the group repeat head G-1: MFMA output rows are independent
     // and those rows are never written out.  No select on the loaded value,
-    // so nothing waits for q before the first page is consumed.
+    // so nothing waits for q before the first tile is consumed.
     const uint16_t *qrow =
         a.q + b * a.q_sb + (int64_t)(h * a.q_group + a.q_off + min(c16, G - 1)) * a.q_sh;
 #pragma unroll
@@ -575,53 +618,70 @@ struct MfmaEngine {
     l_g = 0.f;
   }
 
-  // K loads are plain: one instruction reads 64 bytes of each of 16 rows, so
-  // every 128-byte line is requested by two instructions, and with the
-  // nontemporal hint the line could leave the cache in between (measured:
-  // more HBM fetches, slower).  V loads read whole rows and keep the hint.
-  __device__ __forceinline__ void fetch(const uint16_t *kp, const uint16_t *vp, Page &pg) const {
+  // The rows of the tile at `base` (wave-uniform) into r.  No tile (live
+  // false): nothing is read.  Load i reads rows RPL i + lane / LPR: with
+  // 8-row tiles those past row 7 fold onto rows 0..7 (RPL is a power of two,
+  // so the mask splits).  The lanes of row `newrow` (-1: none) read nothing.
+  template <bool APP>
+  __device__ __forceinline__ void fetch(const uint16_t *base, bool live, int newrow,
+                                        uint4 (&r)[NL]) const {
+    const uint32_t off = voff + (live ? 0u : kRegionSkip);
 #pragma unroll
-    for (int kk = 0; kk < NK; ++kk)
-      pg.k[kk] = *reinterpret_cast<const uint4 *>(kp + koff + 32 * kk);
-    // Load i reads rows RPL i + lane / LPR: with 8-row tiles those past row
-    // 7 fold onto rows 0..7 (RPL is a power of two, so the mask splits).
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      pg.v[i] = stream_load16(vp + voff + ((RPL * i) & rmask) * row_stride);
-  }
-
-  // fetch() for a walk whose sequence appends a token in this launch: the
-  // lanes of row `newrow` of the page (-1: none) read the new token's K/V
-  // (k_row / v_row, this KV head's D elements) instead of the cache.
-  __device__ __forceinline__ void fetch_new(const uint16_t *kp, const uint16_t *vp, Page &pg,
-                                            int newrow, const uint16_t *k_row,
-                                            const uint16_t *v_row) const {
-    const int grp = lane >> 4;
-    const uint16_t *kb = (lane & 15) == newrow ? k_row + 8 * grp : kp + koff;
-#pragma unroll
-    for (int kk = 0; kk < NK; ++kk)
-      pg.k[kk] = *reinterpret_cast<const uint4 *>(kb + 32 * kk);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int t = RPL * i + lane / LPR;
-      pg.v[i] = stream_load16(t == newrow ? v_row + 8 * (lane % LPR)
-                                          : vp + voff + RPL * i * row_stride);
+    for (int i = 0; i < NL; ++i) {
+      uint32_t oi = off;
+      if (APP && RPL * i + lane / LPR == newrow) oi = kRegionSkip;
+      r[i] = region_load16(base, tile_bytes, oi, ((RPL * i) & rmask) * row_bytes);
     }
   }
 
-  // Page score of the walk's KV head from the page's keys, bit for bit the
+  // kr to the K tile, then back in the A operand layout (kop).  The row of a
+  // token appended by this launch (newrow, -1: none) comes from k_new.
+  template <bool APP>
+  __device__ __forceinline__ void stage_k(Lds &lds, int newrow, const uint16_t *k_new) const {
+    uint16_t *dst = &lds.t.k[(lane / LPR) * kRow + 8 * (lane % LPR)];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = kr[i];
+    if (APP && newrow >= 0 && lane < LPR)
+      *reinterpret_cast<uint4 *>(&lds.t.k[newrow * kRow + 8 * lane]) =
+          *reinterpret_cast<const uint4 *>(k_new + 8 * lane);
+  }
+  __device__ __forceinline__ void k_operand(const Lds &lds, uint4 (&kop)[NK]) const {
+    const int c16 = lane & 15, grp = lane >> 4;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+      kop[kk] = *reinterpret_cast<const uint4 *>(&lds.t.k[c16 * kRow + 32 * kk + 8 * grp]);
+  }
+  // vr to the V tile (rows past the context are stored as zeros: the
+  // reference never reads them).
+  template <bool APP>
+  __device__ __forceinline__ void stage_v(Lds &lds, int ntok, int newrow,
+                                          const uint16_t *v_new) {
+    uint16_t *dst = &lds.t.v[(lane / LPR) * kRow + 8 * (lane % LPR)];
+    if (ntok < kPageTokens) {  // uniform: a sequence's last tile, or none
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+        if (RPL * i + lane / LPR >= ntok) vr[i] = make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = vr[i];
+    if (APP && newrow >= 0 && lane < LPR)
+      *reinterpret_cast<uint4 *>(&lds.t.v[newrow * kRow + 8 * lane]) =
+          *reinterpret_cast<const uint4 *>(v_new + 8 * lane);
+  }
+
+  // Page score of the walk's KV head from the tile's keys, bit for bit the
   // page scoring's (score_group_wave): lane (c16, grp) holds dimensions
   // 32 kk + 8 grp .. +8 of token c16, the scorer's segment s = 4 kk + grp,
   // so the scorer's pairwise sum over s (bit 0, 1, 2, 3 of s in turn) is
   // the partner at lane ^ 16, at lane ^ 32, then the kk pairs; the maximum
   // over the ntok valid tokens follows.  qrep: the 16 segments of q_rep.
-  __device__ __forceinline__ float page_score(const Page &pg, int ntok,
+  __device__ __forceinline__ float page_score(const uint4 (&kop)[NK], int ntok,
                                               const uint4 *qrep) const {
     static_assert(NK == 4, "segment mapping of the 128-dimension rows");
     const int grp = lane >> 4;
     float x[NK];
 #pragma unroll
-    for (int kk = 0; kk < NK; ++kk) x[kk] = dot8_bf16(pg.k[kk], qrep[4 * kk + grp], 0.f);
+    for (int kk = 0; kk < NK; ++kk) x[kk] = dot8_bf16(kop[kk], qrep[4 * kk + grp], 0.f);
     float a, b;
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk) {
@@ -642,13 +702,14 @@ struct MfmaEngine {
     return m + 0.f;
   }
 
-  __device__ __forceinline__ void consume(Page &pg, int ntok, Lds &lds) {
-    const int c16 = lane & 15, grp = lane >> 4;
-    const int t0 = 4 * grp;
+  // Scores of the tile and the softmax state: returns P (head c16, tokens
+  // t0 .. t0+3) as bf16 high parts and bf16 remainders.
+  __device__ __forceinline__ bf16x8_t softmax(const uint4 (&kop)[NK], int ntok, Lds &lds) {
+    const int t0 = 4 * (lane >> 4);
     float4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, pg.k[kk]),
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kop[kk]),
                                                     qb[kk], acc, 0, 0, 0);
     float sv[4];
     float pm = -INFINITY;
@@ -661,7 +722,7 @@ struct MfmaEngine {
     xchg16(pm, x, y);
     pm = fmaxf(x, y);
     xchg32(pm, x, y);
-    pm = fmaxf(x, y);  // page max of head c16, in all four of its lanes
+    pm = fmaxf(x, y);  // tile max of head c16, in all four of its lanes
     const float m_new = fmaxf(m_g, pm);
     if (__ballot(m_new > m_g) != 0) {  // some head of the wave rescales
       const float alpha = m_new > m_g ? (m_g == -INFINITY ? 0.f : fast_exp(m_g - m_new)) : 1.f;
@@ -677,38 +738,38 @@ struct MfmaEngine {
         o[blk][3] *= ar.w;
       }
     }
-    // P (head c16, tokens t0 .. t0+3) as bf16 high part + bf16 remainder.
-    short4_t ph, pl;
+    float p[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float p = sv[j] == -INFINITY ? 0.f : fast_exp(sv[j] - m_g);
-      l_g += p;
-      const uint32_t hi = f32_to_bf16_bits(p);
-      const float rem = p - __uint_as_float(hi << 16);
-      ph[j] = (short)hi;
-      pl[j] = (short)f32_to_bf16_bits(rem);
+      p[j] = sv[j] == -INFINITY ? 0.f : fast_exp(sv[j] - m_g);
+      l_g += p[j];
     }
-    // V page -> LDS tile (rows past the context are stored as zeros: the
-    // reference never reads them).
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int t = RPL * i + lane / LPR;
-      const uint4 w = t < ntok ? pg.v[i] : make_uint4(0u, 0u, 0u, 0u);
-      *reinterpret_cast<uint4 *>(&lds.v[t * kVRow + 8 * (lane % LPR)]) = w;
-    }
+    uint4 w;
+    w.x = cvt_bf16x2(p[0], p[1]);
+    w.y = cvt_bf16x2(p[2], p[3]);
+    w.z = cvt_bf16x2(p[0] - bf16_lo(w.x), p[1] - bf16_hi(w.x));
+    w.w = cvt_bf16x2(p[2] - bf16_lo(w.y), p[3] - bf16_hi(w.y));
+    return __builtin_bit_cast(bf16x8_t, w);
+  }
+
+  __device__ __forceinline__ void accumulate(bf16x8_t p, Lds &lds) {
+    const int c16 = lane & 15, t0 = 4 * (lane >> 4);
+    typedef __attribute__((address_space(3))) short4_t lds_short4;
+    // Lane (c16, grp) names row t0 + c16/4, columns 4 (c16 % 4) .. +4 of a
+    // block's 4 x 16 tokens x columns; the transposing read returns it the
+    // four tokens t0 .. t0+3 of column c16.
+    const uint16_t *src = &lds.t.v[(t0 + (c16 >> 2)) * kRow + 4 * (c16 & 3)];
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk) {
-      short4_t vb;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) vb[j] = (short)lds.v[(t0 + j) * kVRow + 16 * blk + c16];
-      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ph, vb, o[blk], 0, 0, 0);
-      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pl, vb, o[blk], 0, 0, 0);
+      const short4_t vb =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(src + 16 * blk));
+      const bf16x8_t vv = __builtin_bit_cast(
+          bf16x8_t, __builtin_shufflevector(vb, vb, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[blk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, vv, o[blk], 0, 0, 0);
     }
   }
 
-  template <int NW>
-  __device__ __forceinline__ void finish(int wave, int lane_, float (*s_o)[G][D],
-                                         float (*s_m)[G], float (*s_l)[G]) {
+  __device__ __forceinline__ void finish(Lds &lds, float *s_m, float *s_l) {
     const int c16 = lane & 15, grp = lane >> 4;
     float x, y;
     xchg16(l_g, x, y);
@@ -716,18 +777,88 @@ struct MfmaEngine {
     xchg32(l_g, x, y);
     l_g = x + y;  // head c16's l over all 16 token rows
     if (lane < G) {
-      s_m[wave][lane] = m_g;
-      s_l[wave][lane] = l_g;
+      s_m[lane] = m_g;
+      s_l[lane] = l_g;
     }
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int g = 4 * grp + j;
-        if (g < G) s_o[wave][g][16 * blk + c16] = o[blk][j];
+        if (g < G) lds.o[g * D + 16 * blk + c16] = o[blk][j];
       }
   }
 };
+
+// Tiles of a chunk of up to 64 of a wave's walk: lane j holds tile j's
+// physical tile and logical tile (kNoTile: none, nothing is read).
+struct TileChunk {
+  int phys = 0, lt = kNoTile;
+};
+
+// One wave's walk over npw tiles.  `cur` is the first chunk's tiles, whose
+// first tile's loads are in flight (start_walk); chunk c's tiles come from
+// lookup(c) while chunk c - 1 is walked, so the loads run on across chunks.
+// score(lt, ntok, kop) sees each tile's keys first (SCORE).  APP: row new_off
+// of logical tile new_tile is the appended token's (k_new / v_new).
+template <class Engine, bool APP>
+__device__ __forceinline__ void fetch_tile(const DecodeArgs &a, const Engine &eng, int phys,
+                                           int lt, int newrow, const uint16_t *cache,
+                                           uint4 (&r)[Engine::NL]) {
+  const int64_t base = (int64_t)phys * (eng.tile_bytes / 2);
+  eng.template fetch<APP>(cache + base, lt != kNoTile, newrow, r);
+}
+
+template <class Engine, bool APP = false>
+__device__ __forceinline__ void start_walk(const DecodeArgs &a, Engine &eng, const TileChunk &cur,
+                                           int new_tile = -1, int new_off = -1) {
+  const int phys = __builtin_amdgcn_readlane(cur.phys, 0);
+  const int lt = __builtin_amdgcn_readlane(cur.lt, 0);
+  const int newrow = APP && lt == new_tile ? new_off : -1;
+  // K before V, here and in the walk: the wait for a tile's K then leaves its
+  // V in flight.
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.k_cache, eng.kr);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.v_cache, eng.vr);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <class Engine, bool APP, bool SCORE, class Lookup, class Score>
+__device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int npw, int ctx,
+                                           TileChunk cur, Lookup lookup, Score score,
+                                           typename Engine::Lds &lds, int new_tile = -1,
+                                           int new_off = -1, const uint16_t *k_new = nullptr,
+                                           const uint16_t *v_new = nullptr) {
+  const int tl = Engine::tlog(a);
+  TileChunk nxt;
+  int lt = __builtin_amdgcn_readlane(cur.lt, 0);
+  for (int e = 0; e < npw; ++e) {
+    const int j = e & (kWave - 1);
+    if (j == 0 && e + kWave < npw) nxt = lookup(e + kWave);
+    if (j == kWave - 1) {  // the next tile is the next chunk's first
+      cur = nxt;
+      nxt = TileChunk();
+    }
+    // Lanes past the walk's end hold no tile.
+    const int phys_n = __builtin_amdgcn_readlane(cur.phys, (j + 1) & (kWave - 1));
+    const int lt_n = __builtin_amdgcn_readlane(cur.lt, (j + 1) & (kWave - 1));
+    const int newrow = APP && lt == new_tile ? new_off : -1;
+    const int newrow_n = APP && lt_n == new_tile ? new_off : -1;
+    const int ntok = min(1 << tl, max(0, ctx - (lt << tl)));
+    eng.template stage_k<APP>(lds, newrow, k_new);
+    fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.k_cache, eng.kr);
+    uint4 kop[Engine::NK];
+    eng.k_operand(lds, kop);
+    if constexpr (SCORE) score(lt, ntok, kop);
+    const bf16x8_t p = eng.softmax(kop, ntok, lds);
+    eng.template stage_v<APP>(lds, ntok, newrow, v_new);
+    fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr);
+    __builtin_amdgcn_sched_barrier(0);
+    eng.accumulate(p, lds);
+    lt = lt_n;
+  }
+}
 
 // The split hand-off's three steps.  publish_partials: every thread's
 // partial-row stores complete before the workgroup's counter moves;
@@ -757,11 +888,22 @@ __device__ __forceinline__ void acquire_partials() {
 #endif
 }
 
-template <class L, int NW>
-__device__ __forceinline__ L &s_eng_of(L (&eng)[NW], int wave) { return eng[wave]; }
+// LDS of a workgroup's page walk and epilogue: the waves' engines (their
+// tiles, then their o), reused by the merge once the workgroup's partial is
+// stored; the waves' (m, l); the last-arriver flag.
+template <int G, class Engine, int NW>
+struct WalkLds {
+  union {
+    typename Engine::Lds eng[NW];
+    MergeLds<G, NW * kWave> merge;
+  } __attribute__((aligned(16)));
+  float m[NW][G];
+  float l[NW][G];
+  int last;
+};
 
 // End of one workgroup's walk over pages of head h (the waves' states are in
-// s_o / s_m / s_l, behind a barrier).  If the workgroup is the head's only
+// lds, behind a barrier).  If the workgroup is the head's only
 // contributor (n_act == 1) it writes the outputs.  Otherwise it stores its
 // partial (o, m, l) in partial row my_row, bumps the head's counter, and the
 // last of the n_act contributors merges rows first_row .. first_row+n_act-1.
@@ -773,15 +915,18 @@ __device__ __forceinline__ L &s_eng_of(L (&eng)[NW], int wave) { return eng[wave
 // rows and writes the outputs.  One workgroup merging ~140 partials takes
 // ~9 dependent batches of loads; two levels take one batch each and one more
 // store-wait-counter.
-template <int G, int D, int NW, int KB, bool TWO = false>
+template <int G, class Engine, int NW, bool TWO = false>
 __device__ __forceinline__ void segment_epilogue(const DecodeArgs &a, const PartBuf &pb, int h,
                                                  int n, int nv, int n_act, uint32_t my_row,
                                                  uint32_t first_row,
-                                                 const float (&s_o)[NW][G][D],
-                                                 const float (&s_m)[NW][G],
-                                                 const float (&s_l)[NW][G], int &s_last,
-                                                 MergeLds<G, NW * kWave> &s_merge) {
+                                                 WalkLds<G, Engine, NW> &lds) {
+  constexpr int D = Engine::kD;
   constexpr int NT = NW * kWave;
+  constexpr int KMAX = TWO ? 8 : 16;
+  auto &s_m = lds.m;
+  auto &s_l = lds.l;
+  auto &s_last = lds.last;
+  auto &s_merge = lds.merge;
   constexpr int kChunksPerRow = D / 4;
   constexpr int kPartStride = part_stride(D);
   // Workgroup state of float4 chunk c (q-head g = c / (D/4), elements d0 .. d0+3):
@@ -799,7 +944,7 @@ __device__ __forceinline__ void segment_epilogue(const DecodeArgs &a, const Part
         const float mw = s_m[wv][g];
         if (mw != -INFINITY) {
           const float f = fast_exp(mw - M);
-          O += f * *reinterpret_cast<const f32x4 *>(&s_o[wv][g][d0]);
+          O += f * *reinterpret_cast<const f32x4 *>(&lds.eng[wv].o[g * D + d0]);
           L += s_l[wv][g] * f;
         }
       }
@@ -842,7 +987,7 @@ __device__ __forceinline__ void segment_epilogue(const DecodeArgs &a, const Part
     if (threadIdx.x == 0)
       __hip_atomic_store(gc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t grow = (first_row + (uint32_t)g0) * kRowElems;
-    merge_partials<G, D, NT, KB, true>(a, pb, grow, gsize, h, 0, 0, s_merge, 1, grow);
+    merge_partials<G, D, NT, KMAX, true>(a, pb, grow, gsize, h, 0, 0, s_merge, 1, grow);
     publish_partials();
     if (threadIdx.x == 0) s_last = handoff_count(&a.counters[h]) == (unsigned)(ng - 1);
     __syncthreads();
@@ -850,7 +995,7 @@ __device__ __forceinline__ void segment_epilogue(const DecodeArgs &a, const Part
       acquire_partials();
       if (threadIdx.x == 0)
         __hip_atomic_store(&a.counters[h], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      merge_partials<G, D, NT, KB>(a, pb, first_row * kRowElems, ng, h, n, nv, s_merge,
+      merge_partials<G, D, NT, KMAX>(a, pb, first_row * kRowElems, ng, h, n, nv, s_merge,
                                    kMergeGroup);
     }
     return;
@@ -862,25 +1007,9 @@ __device__ __forceinline__ void segment_epilogue(const DecodeArgs &a, const Part
     // Last contributor of the head: merge its partials, write the outputs.
     if (threadIdx.x == 0)
       __hip_atomic_store(&a.counters[h], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    merge_partials<G, D, NT, KB>(a, pb, first_row * kRowElems, n_act, h, n, nv, s_merge);
+    merge_partials<G, D, NT, KMAX>(a, pb, first_row * kRowElems, n_act, h, n, nv, s_merge);
   }
 }
-
-// LDS of a workgroup's page walk and epilogue: the waves' (o, m, l), the
-// last-arriver flag, and the engines' LDS, which is dead once a walk ends and
-// is reused by the merge.
-template <int G, class Engine, int NW>
-struct WalkLds {
-  union Tail {
-    typename Engine::Lds eng[NW];
-    MergeLds<G, NW * kWave> merge;
-  };
-  float o[NW][G][Engine::kD] __attribute__((aligned(16)));
-  float m[NW][G];
-  float l[NW][G];
-  int last;
-  Tail tail __attribute__((aligned(16)));
-};
 
 // The first page-list entries of split `split` of head bh (lane j of wave
 // w: entry r0 + w + NW j) and their block-table entries, requested as early
@@ -943,13 +1072,12 @@ __device__ __forceinline__ int listed_pps(const DecodeArgs &a, int n, int ts) {
 // With SCORE and a.spec_scores, the walk also writes the page score of
 // every page it walks (Engine::page_score; qrep: this wave's LDS copy of the
 // 16 q_rep segments, 16-token pages).
-template <int G, class Engine, int NW, int PD, bool APP = false, bool SCORE = false,
+template <int G, class Engine, int NW, bool APP = false, bool SCORE = false,
           bool IDENT = false>
 __device__ __forceinline__ void listed_walk(const DecodeArgs &a, int split, int bh, int spec_lp,
                                             int spec_phys, WalkLds<G, Engine, NW> &L,
                                             const NewToken &nt = NewToken(),
                                             uint4 *qrep = nullptr) {
-  using Page = typename Engine::Page;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = bh / a.H_kv;
@@ -975,96 +1103,67 @@ __device__ __forceinline__ void listed_walk(const DecodeArgs &a, int split, int 
   if (r0 >= r1 && !(split == 0 && n_act == 0)) return;  // uniform
 
   Engine eng;
-  eng.init(a, b, h, lane, s_eng_of(L.tail.eng, wave));
+  eng.init(a, b, h, lane);
   // Wave-private q_rep: lane < 16 computes segment `lane` (its loads go out
-  // ahead of the first pages') and stores it to LDS just before the first
-  // page score, so no wait for q holds up the first page requests; the LDS
-  // store and the later reads are the same wave's, in order.
+  // ahead of the first tile's) and stores it to LDS once the first tile is
+  // requested; the LDS store and the later reads are the same wave's, in
+  // order.
   const bool scoring = SCORE && a.spec_scores != nullptr;  // uniform
   uint4 qr_own = make_uint4(0u, 0u, 0u, 0u);
-  bool qr_stored = false;
   if constexpr (SCORE) {
     if (scoring)
       qr_own = group_mean_q(a.q, a.q_sb, a.q_sh, b, h, a.q_group, min(lane, 15), a.inv_g);
   }
-  const int64_t page_elems = ((int64_t)a.H_kv * Engine::kD) << tl;  // between tiles
   const int npw = max(0, (r1 - r0 - wave + NW - 1) / NW);
-  for (int c0 = 0; c0 < npw; c0 += kWave) {
-    const int cn = min(kWave, npw - c0);
-    int my_phys = 0, my_ntok = 0, my_new = -1, my_lt = -1;
-    if (lane < cn) {
-      const bool spec = c0 == 0 && !refetch;
-      const int lt = spec ? spec_lp
-                     : IDENT ? r0 + wave + NW * (c0 + lane)
-                             : listed_tile(a, idx_row, r0 + wave + NW * (c0 + lane), ts);
-      if (lt >= 0 && lt < (a.W << ts)) {
-        my_lt = lt;
-        int pt = spec ? spec_phys : tile_block(a, b, lt, ts);
-        if (APP && lt == nt.page && nt.new_blk >= 0) pt = nt.new_blk;
-        if (pt >= 0 && pt < (a.num_blocks << ts)) {
-          my_phys = pt;
-          my_ntok = max(0, min(1 << tl, ctx - (lt << tl)));
-          if (APP && lt == nt.page) my_new = nt.off;
-        }
-      }
+  // Tile `lane` of the chunk that starts at the wave's tile c0: its entry's
+  // logical tile and that tile's physical one, if both are valid.
+  auto chunk = [&](int c0, int lt, int phys) {
+    TileChunk c;
+    if (APP && lt == nt.page && nt.new_blk >= 0) phys = nt.new_blk;
+    if (c0 + lane < npw && lt >= 0 && lt < (a.W << ts) && phys >= 0 &&
+        phys < (a.num_blocks << ts)) {
+      c.phys = phys;
+      c.lt = lt;
     }
-    // Loads are unconditional so that no branch separates a prefetch from
-    // the page being consumed: a page without valid tokens reads block 0 (in
-    // bounds) and is masked out by consume(); prefetches past the end re-read
-    // the wave's last page (already cached) and are never consumed.
-    auto fetch = [&](int j, Page &pg) {
-      const int64_t base = (int64_t)__builtin_amdgcn_readlane(my_phys, j) * page_elems;
-      if constexpr (APP)
-        eng.fetch_new(a.k_cache + base, a.v_cache + base, pg,
-                      __builtin_amdgcn_readlane(my_new, j), nt.k, nt.v);
-      else
-        eng.fetch(a.k_cache + base, a.v_cache + base, pg);
-      return __builtin_amdgcn_readlane(my_ntok, j);
-    };
-    Page pbuf[PD];
-    int nt[PD];
-    // The first trip fetches pages 0..PD-1 and consumes page 0; every fetch
-    // of a slot uses the same registers and the wait counts see PD-1 pages
-    // outstanding.
-    for (int j = 1 - PD; j < cn; j += PD) {
-#pragma unroll
-      for (int u = 0; u < PD; ++u) {
-        const int slot = (u + PD - 1) % PD;  // slot of page j+u+PD-1
-        nt[slot] = fetch(min(j + u + PD - 1, cn - 1), pbuf[slot]);
-        if (j + u >= 0 && j + u < cn) {
-          if constexpr (SCORE) {
-            if (scoring) {
-              if (!qr_stored) {
-                if (lane < 16) qrep[lane] = qr_own;
-                qr_stored = true;
-              }
-              const float sc = eng.page_score(pbuf[u], nt[u], qrep);
-              const int lt = __builtin_amdgcn_readlane(my_lt, j + u);
-              if (lane == 0 && lt >= 0) a.spec_scores[(int64_t)bh * a.W + lt] = sc;
-            }
-          }
-          eng.consume(pbuf[u], nt[u], s_eng_of(L.tail.eng, wave));
-        }
-      }
-    }
+    return c;
+  };
+  auto lookup = [&](int c0) {
+    const int e = r0 + wave + NW * min(c0 + lane, max(npw - 1, 0));
+    const int lt = IDENT ? e : listed_tile(a, idx_row, e, ts);
+    return chunk(c0, lt, tile_block(a, b, lt, ts));
+  };
+  const TileChunk first = refetch && npw > 0 ? lookup(0) : chunk(0, spec_lp, spec_phys);
+  start_walk<Engine, APP>(a, eng, first, nt.page, nt.off);
+  if constexpr (SCORE) {
+    if (scoring && lane < 16) qrep[lane] = qr_own;
   }
-  eng.template finish<NW>(wave, lane, L.o, L.m, L.l);
+  walk_tiles<Engine, APP, SCORE>(
+      a, eng, npw, ctx, first, lookup,
+      [&](int lt, int ntok, const uint4 (&kop)[Engine::NK]) {
+        if constexpr (SCORE) {
+          if (scoring) {
+            const float sc = eng.page_score(kop, ntok, qrep);
+            if (lane == 0 && lt != kNoTile) a.spec_scores[(int64_t)bh * a.W + lt] = sc;
+          }
+        }
+      },
+      L.eng[wave], nt.page, nt.off, nt.k, nt.v);
+  eng.finish(L.eng[wave], L.m[wave], L.l[wave]);
   __syncthreads();
   const PartBuf pb(a.part, a.part_bytes);
-  segment_epilogue<G, Engine::kD, NW, kMergeBatchListed>(
-      a, pb, bh, n >> ts, valid_pages_sh(ctx, tl + ts), n_act, (uint32_t)(bh * n_spl + split),
-      (uint32_t)(bh * n_spl), L.o, L.m, L.l, L.last, L.tail.merge);
+  segment_epilogue<G, Engine, NW>(a, pb, bh, n >> ts, valid_pages_sh(ctx, tl + ts), n_act,
+                                  (uint32_t)(bh * n_spl + split), (uint32_t)(bh * n_spl), L);
 }
 
 // The listed decode: a static grid of (split, head) workgroups.
-template <int G, class Engine, int NW, int PD>
-__global__ __launch_bounds__(NW * kWave) void listed_decode_kernel(const DecodeArgs a) {
+template <int G, class Engine, int NW>
+__global__ __launch_bounds__(NW * kWave, walk_waves(Engine::kD)) void listed_decode_kernel(const DecodeArgs a) {
   __shared__ WalkLds<G, Engine, NW> L;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int lp, phys;
   listed_first_pages<NW>(a, blockIdx.x, blockIdx.y, wave, lane, Engine::tshift(a), lp, phys);
-  listed_walk<G, Engine, NW, PD>(a, blockIdx.x, blockIdx.y, lp, phys, L);
+  listed_walk<G, Engine, NW>(a, blockIdx.x, blockIdx.y, lp, phys, L);
 }
 
 // The listed decode of a reuse step with the step's token append folded in
@@ -1075,8 +1174,8 @@ __global__ __launch_bounds__(NW * kWave) void listed_decode_kernel(const DecodeA
 // sequence's first head also moves its context length, page-table entry
 // and allocation count as cvsa_append_kv does.  Later launches see the
 // appended cache.
-template <int G, class Engine, int NW, int PD>
-__global__ __launch_bounds__(NW * kWave) void listed_append_kernel(const DecodeArgs a,
+template <int G, class Engine, int NW>
+__global__ __launch_bounds__(NW * kWave, walk_waves(Engine::kD)) void listed_append_kernel(const DecodeArgs a,
                                                                    const AppendArgs app) {
   static_assert(Engine::kD == 128, "the fused append is built for D = 128");
   __shared__ WalkLds<G, Engine, NW> L;
@@ -1099,32 +1198,31 @@ __global__ __launch_bounds__(NW * kWave) void listed_append_kernel(const DecodeA
   listed_first_pages<NW>(a, split, bh, wave, lane, 0, lp, phys);
   if (lp == nt.page && nt.new_blk >= 0) phys = nt.new_blk;
   // Split 0's wave 0 appends: lanes 0-15 copy the head's K row, lanes 16-31
-  // its V row, 16 bytes each.  Their loads are requested with the walk's
-  // first ones and the stores wait until the walk is done.
+  // its V row, 16 bytes each.  No workgroup of the launch reads the slot, the
+  // context length or the new page's table entry, so the stores go out at
+  // once, behind the walk's first lookups.
   const bool writer = ok && split == 0 && wave == 0;  // uniform
-  int blk = -1;
-  uint4 x = make_uint4(0u, 0u, 0u, 0u);
   if (writer) {
-    blk = nt.new_blk >= 0 ? nt.new_blk : a.block_tables[(int64_t)b * a.bt_sb + nt.page];
-    x = *reinterpret_cast<const uint4 *>((lane >= 16 ? nt.v : nt.k) + 8 * (lane & 15));
+    const int blk =
+        nt.new_blk >= 0 ? nt.new_blk : a.block_tables[(int64_t)b * a.bt_sb + nt.page];
+    const uint4 x = *reinterpret_cast<const uint4 *>((lane >= 16 ? nt.v : nt.k) + 8 * (lane & 15));
+    if (lane < 32 && blk >= 0 && blk < a.num_blocks) {
+      const int64_t dst =
+          (((int64_t)blk * kPageTokens + nt.off) * a.H_kv + h) * Engine::kD + 8 * (lane & 15);
+      *reinterpret_cast<uint4 *>(const_cast<uint16_t *>(lane >= 16 ? a.v_cache : a.k_cache) +
+                                 dst) = x;
+    }
+    if (h == 0 && lane == 0) {
+      app.ctx_lens[b] = sl.x + 1;
+      if (nt.new_blk >= 0) {
+        app.block_tables[(int64_t)b * a.bt_sb + nt.page] = nt.new_blk;
+        app.pages_allocated[b] += 1;
+      }
+    }
   }
   if (!ok && split == 0 && h == 0 && threadIdx.x == 0 && app.slot_errors != nullptr)
     atomicAdd(app.slot_errors, 1);  // a rejected device slot is reported, not dropped silently
-  listed_walk<G, Engine, NW, PD, true>(a, split, bh, lp, phys, L, nt);
-  if (!writer) return;
-  if (lane < 32 && blk >= 0 && blk < a.num_blocks) {
-    const int64_t dst =
-        (((int64_t)blk * kPageTokens + nt.off) * a.H_kv + h) * Engine::kD + 8 * (lane & 15);
-    *reinterpret_cast<uint4 *>(const_cast<uint16_t *>(lane >= 16 ? a.v_cache : a.k_cache) +
-                               dst) = x;
-  }
-  if (h == 0 && lane == 0) {
-    app.ctx_lens[b] = sl.x + 1;
-    if (nt.new_blk >= 0) {
-      app.block_tables[(int64_t)b * a.bt_sb + nt.page] = nt.new_blk;
-      app.pages_allocated[b] += 1;
-    }
-  }
+  listed_walk<G, Engine, NW, true>(a, split, bh, lp, phys, L, nt);
 }
 
 // 16-token tiles per scoring wave of the fused launch below.
@@ -1151,18 +1249,13 @@ constexpr int kSpecHeadPPW = 16;
 // kernel, rewrites.
 // One launch lets the decode's dependent metadata loads and split hand-off
 // overlap the scoring stream without a second stream and its events.
-// Three waves per SIMD (the register budget that allows, 168 VGPRs, holds
-// the decode without spills): 768 workgroups resident instead of 512, so the
-// decode and scoring workgroups of a cfg3 launch all run at once (check
-// step 68.4 -> 64.5 us at cfg3, 82.2 -> 75.5 us at cfg4).  Reading the kept
-// selection's keys once: kept check 64.0 -> 61.1 us at cfg3 (16 pages per
-// scoring wave; 8 and 32 measured 61.2 and 62.0).
-template <int G, class Engine, int NW, int PD>
-__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(3)))
-void score_spec_kernel(const DecodeArgs a,
-                                                                const ScoreArgs s,
-                                                                int score_gx) {
-  static_assert(NW == 4, "the scoring part runs four waves per workgroup");
+// Up to four waves per SIMD (128 registers; groups above 8 would spill there
+// and take 168): the decode and scoring workgroups of a cfg3 launch all run
+// at once.  Reading the kept selection's keys once: kept check 64.0 -> 61.1 us
+// at cfg3 (16 pages per scoring wave; 8 and 32 measured 61.2 and 62.0).
+template <int G, class Engine, int NW>
+__global__ __launch_bounds__(NW * kWave, Engine::kTileShift != 0 ? 2 : G > 8 ? 3 : 4)
+void score_spec_kernel(const DecodeArgs a, const ScoreArgs s, int score_gx) {
   __shared__ WalkLds<G, Engine, NW> L;
   __shared__ uint4 s_qrep[NW][16];  // decode part: q_rep per wave
   const int lane = threadIdx.x & 63;
@@ -1197,7 +1290,7 @@ void score_spec_kernel(const DecodeArgs a,
     const int bh = w / a.n_splits;
     int lp, phys;
     listed_first_pages<NW>(a, split, bh, wave, lane, Engine::tshift(a), lp, phys);
-    listed_walk<G, Engine, NW, PD, false, Engine::kTileShift == 0>(a, split, bh, lp, phys, L,
+    listed_walk<G, Engine, NW, false, Engine::kTileShift == 0>(a, split, bh, lp, phys, L,
                                                                    NewToken(), s_qrep[wave]);
   } else if constexpr (Engine::kTileShift == 0) {
     if (go != 2 || w >= a.n_splits_all * a.heads) return;  // uniform
@@ -1205,13 +1298,11 @@ void score_spec_kernel(const DecodeArgs a,
     const int bh = w / a.n_splits_all;
     int lp, phys;
     ident_first_pages<NW>(a, split, bh, wave, lane, 0, lp, phys);
-    listed_walk<G, Engine, NW, PD, false, true, true>(a, split, bh, lp, phys, L, NewToken(),
+    listed_walk<G, Engine, NW, false, true, true>(a, split, bh, lp, phys, L, NewToken(),
                                                       s_qrep[wave]);
   }
 }
 
-// NW waves per workgroup, PD pages of K/V in flight per wave.
-//
 // Every workgroup first computes the pages each head walks and their prefix
 // (the same partition in every workgroup), then walks the segments of its
 // range: (head h, pages s0..s1 of h's walk).  A segment that is a whole head
@@ -1221,24 +1312,16 @@ void score_spec_kernel(const DecodeArgs a,
 // consecutive rows owner(first page) + h .. owner(last page) + h), bumps the
 // head's counter, and the last contributor merges.  Heads that walk no pages
 // are written by workgroup h mod n_wg.
-template <int G, class Engine, int NW, int PD, int MODE>
-__global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const DecodeArgs a) {
+template <int G, class Engine, int NW, int MODE>
+__global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_decode_kernel(
+    const DecodeArgs a) {
   constexpr int NT = NW * kWave;         // threads per workgroup
-  static_assert(NW == 4, "kMinPagesPerWg assumes four waves");
-  using Page = typename Engine::Page;
 
   __shared__ WalkLds<G, Engine, NW> L;
   __shared__ int s_wsum[NW];
   __shared__ int s_odd[NW];               // a head of the wave's pass walks != max_sel pages
   __shared__ int s_start[kMaxHeads + 1];  // exclusive prefix of pages per head
   __shared__ uint8_t s_listed[kMaxHeads];  // kWalk* of each head
-  auto &s_o = L.o;
-  auto &s_m = L.m;
-  auto &s_l = L.l;
-  auto &s_last = L.last;
-  auto &s_tail = L.tail;
-  auto &s_eng = s_tail.eng;
-
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int w = blockIdx.x;
@@ -1246,7 +1329,6 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
   constexpr int D = Engine::kD;
   const int ts = Engine::tshift(a);
   const int tl = Engine::tlog(a);
-  const int64_t page_elems = ((int64_t)a.H_kv * D) << tl;  // between tiles
 
   // Verified launches whose heads are all accepted (a lazy check that keeps
   // its selection, or a scoring step whose gate passes everywhere) run the
@@ -1279,7 +1361,7 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
     accepted = __syncthreads_or(accepted);
     if (rejected == 0) {  // uniform
       if (w < n_listed)
-        listed_walk<G, Engine, NW, PD>(a, split, bh, lp,
+        listed_walk<G, Engine, NW>(a, split, bh, lp,
                                        listed_first_block(a, bh, lp, Engine::tshift(a)), L);
       return;
     }
@@ -1306,7 +1388,7 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
       const int ibh = w / a.n_splits_all;
       int ilp, iphys;
       ident_first_pages<NW>(a, isplit, ibh, wave, lane, ts, ilp, iphys);
-      listed_walk<G, Engine, NW, PD, false, false, true>(a, isplit, ibh, ilp, iphys, L);
+      listed_walk<G, Engine, NW, false, false, true>(a, isplit, ibh, ilp, iphys, L);
       return;
     }
   }
@@ -1315,8 +1397,8 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
   // max_sel listed pages: the range start is then known without the scan.
   // The first page-list entries, the head's context length and q and the
   // head counts of the scan are requested at entry, the pages' block-table
-  // entries as soon as the page-list entries arrive, and the first PD pages
-  // of K/V before the scan: two memory round trips fewer before the first
+  // entries as soon as the page-list entries arrive, and the first tile of
+  // K/V before the scan: two memory round trips fewer before the first
   // K/V load.  Used only if the scan confirms the case.  The loads are
   // issued without branches (indices clamped; a WG without a speculated
   // range reads harmless in-bounds entries and discards them), so the
@@ -1342,7 +1424,7 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
     const int lp0 = *src;
     spec_lp = ts == 0 ? lp0 : lp0 >= 0 && lp0 < a.W ? (lp0 << ts) | (rs & ((1 << ts) - 1)) : -1;
     ctx_spec = __builtin_amdgcn_readfirstlane(a.ctx_lens[b_spec]);
-    eng.init(a, b_spec, hs - b_spec * a.H_kv, lane, s_eng[wave]);
+    eng.init(a, b_spec, hs - b_spec * a.H_kv, lane);
     if (a.max_sel > 0 && w < spec_part.n) h_spec = hs;
   }
 
@@ -1363,67 +1445,35 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
       __ballot((int)threadIdx.x < heads && (c_first != max_sel_t || l_first == kWalkAlt)) != 0;
   if (lane == 0) s_odd[wave] = odd_first ? 1 : 0;
 
-  // One wave's walk over its pages s0 + wave + NW*j of a segment, in chunks
-  // of up to 64 pages: lane j of a chunk looks up page j's block id and
-  // valid-token count; the loop reads them with readlane and keeps PD pages
-  // of K/V loads in flight (slot (u + PD - 1) % PD holds page u after the
-  // prologue).  Loads are unconditional so that no branch separates a
-  // prefetch from the page being consumed: a page without valid tokens reads
-  // block 0 (in bounds) and is masked out by consume(); prefetches past the
-  // end re-read the wave's last page (already cached) and are never consumed.
-  Page pbuf[PD];
-  int nt[PD];                 // logical page of each slot (kNoPage: none)
-  int my_phys = 0, my_lp = 0;
-  int cur_ctx = 0;            // context length of the segment being walked
-  constexpr int kNoPage = 1 << 26;  // ctx - kNoPage * 16 < 0: no valid token
-  auto lookup = [&](int s0, int c0, int cn, bool listed, const int32_t *idx_row, int b,
+  // Tiles c0 .. of a wave's part of a segment (its tiles s0 + wave + NW j,
+  // j < npw), one per lane; `spec` takes the speculative entries.
+  auto lookup = [&](int s0, int c0, int npw, bool listed, const int32_t *idx_row, int b,
                     bool spec) {
-    const int r = s0 + wave + NW * (c0 + lane);
+    const int r = s0 + wave + NW * min(c0 + lane, max(npw - 1, 0));
     int lp = r, phys = 0;
-    if (spec) {  // the speculative entries of the chunk (tile of entry r), consumed by every lane
+    if (spec) {
       lp = spec_lp;
       phys = spec_phys;
-    } else if (lane < cn) {
+    } else if (npw > 0) {
       if (listed) lp = listed_tile(a, idx_row, r, ts);
       phys = tile_block(a, b, lp, ts);
     }
-    const bool ok = lane < cn && lp >= 0 && lp < (a.W << ts) && phys >= 0 &&
-                    phys < (a.num_blocks << ts);
-    my_phys = ok ? phys : 0;
-    my_lp = ok ? lp : kNoPage;
-  };
-  // Page j of the chunk into pg; returns its logical page (the valid-token
-  // count needs the context length only when the page is consumed).
-  auto fetch = [&](int j, Page &pg) {
-    const int64_t base = (int64_t)__builtin_amdgcn_readlane(my_phys, j) * page_elems;
-    eng.fetch(a.k_cache + base, a.v_cache + base, pg);
-    return __builtin_amdgcn_readlane(my_lp, j);
-  };
-  auto ntok = [&](int lp) { return min(1 << tl, max(0, cur_ctx - (lp << tl))); };
-  auto prologue = [&](int cn) {
-#pragma unroll
-    for (int u = 0; u < PD; ++u)
-      nt[(u + PD - 1) % PD] = fetch(max(0, min(u, cn - 1)), pbuf[(u + PD - 1) % PD]);
-  };
-  auto steady = [&](int cn) {
-    eng.consume(pbuf[PD - 1], ntok(nt[PD - 1]), s_eng[wave]);  // page 0
-    for (int j = 1; j < cn; j += PD) {
-#pragma unroll
-      for (int u = 0; u < PD; ++u) {
-        const int slot = (u + PD - 1) % PD;  // slot of page j+u+PD-1
-        nt[slot] = fetch(min(j + u + PD - 1, cn - 1), pbuf[slot]);
-        if (j + u < cn) eng.consume(pbuf[u], ntok(nt[u]), s_eng[wave]);
-      }
+    TileChunk c;
+    if (c0 + lane < npw && lp >= 0 && lp < (a.W << ts) && phys >= 0 &&
+        phys < (a.num_blocks << ts)) {
+      c.phys = phys;
+      c.lt = lp;
     }
+    return c;
   };
 
-  // First PD pages of the speculated segment (a WG without one fetches block
-  // 0 and never consumes it).
+  // First tile of the speculated segment (a WG without one reads nothing).
+  TileChunk first;
   if constexpr (MODE != kModeAll) {
     const int s1 = min(g1_spec, (h_c + 1) * max_sel_t) - h_c * max_sel_t;
     const int npw = h_spec >= 0 ? max(0, (s1 - r_spec - wave + NW - 1) / NW) : 0;
-    lookup(r_spec, 0, min(kWave, npw), true, nullptr, b_spec, true);
-    prologue(min(kWave, npw));
+    first = lookup(r_spec, 0, npw, true, nullptr, b_spec, true);
+    start_walk<Engine>(a, eng, first);
   }
   // Pass 0 (peeled: a loop header here makes the compiler wait for the
   // speculative loads), then the passes of launches with more than NT heads.
@@ -1517,26 +1567,25 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
                                  : a.page_idx + (int64_t)h * a.idx_stride;
     const bool use_spec = spec_ok && on_spec && s0 == r_spec && walk == kWalkListed;
 
-    if (!on_spec || h != lo) eng.init(a, b, hk, lane, s_eng[wave]);
-    cur_ctx = ctx;
+    if (!on_spec || h != lo) eng.init(a, b, hk, lane);
     const int npw = max(0, (s1 - s0 - wave + NW - 1) / NW);
-    for (int c0 = 0; c0 < npw; c0 += kWave) {
-      const int cn = min(kWave, npw - c0);
-      if (!(use_spec && c0 == 0)) {  // the speculated chunk is already in flight
-        lookup(s0, c0, cn, listed, idx_row, b, false);
-        prologue(cn);
-      }
-      steady(cn);
+    if (!use_spec) {  // else the speculated first tile is already in flight
+      first = lookup(s0, 0, npw, listed, idx_row, b, false);
+      start_walk<Engine>(a, eng, first);
     }
-    eng.template finish<NW>(wave, lane, s_o, s_m, s_l);
+    walk_tiles<Engine, false, false>(
+        a, eng, npw, ctx, first,
+        [&](int c0) { return lookup(s0, c0, npw, listed, idx_row, b, false); },
+        [](int, int, const uint4 (&)[Engine::NK]) {}, L.eng[wave]);
+    eng.finish(L.eng[wave], L.m[wave], L.l[wave]);
     __syncthreads();
 
-    const int first = part.owner(P);
+    const int first_wg = part.owner(P);
     const int nv = valid_pages_sh(ctx, tl + ts);
     const int booked = MODE == kModeApprox ? approx_booked_pages(a, h, nv) : n >> ts;
-    segment_epilogue<G, D, NW, kMergeBatchStreamK, true>(a, pb, h, booked, nv,
-                               part.owner(P + n - 1) - first + 1, (uint32_t)(w + h),
-                               (uint32_t)(first + h), s_o, s_m, s_l, s_last, s_tail.merge);
+    segment_epilogue<G, Engine, NW, true>(a, pb, h, booked, nv,
+                                          part.owner(P + n - 1) - first_wg + 1,
+                                          (uint32_t)(w + h), (uint32_t)(first_wg + h), L);
     __syncthreads();  // LDS is reused by the next segment
   }
 }
@@ -1545,58 +1594,55 @@ __global__ __launch_bounds__(NW * kWave) void streamk_decode_kernel(const Decode
 // in one workgroup's LDS): one per CU of the 256-CU part.
 constexpr int kTargetWorkgroups = 256;
 static_assert(kTargetWorkgroups <= kMaxSplits, "one merge per head fits the merge LDS");
-constexpr int kWavesPerWg = 4;
 
 // Launches of a validated decode for GQA group size G, explicitly
 // instantiated per G in the decode_g*.hip files (one translation unit per
-// four group sizes, so the library's objects compile in parallel).  Pages of
-// K/V in flight per wave: 2, or 1 at D = 256, whose pages hold twice the
-// registers.
+// four group sizes, so the library's objects compile in parallel). 
 enum { kLaunchListed = 0, kLaunchVerified = 1, kLaunchAll = 2, kLaunchApprox = 3 };
 
 template <int G, int D, int TS>
-void launch_decode_gdt(const DecodeArgs &a, int kind, dim3 grid, dim3 block, hipStream_t st) {
-  constexpr int PD = D > 128 ? 1 : 2;
+void launch_decode_gdt(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
+  const dim3 block(kWavesPerWg * kWave);
   using E = MfmaEngine<G, D, TS>;
   if (kind == kLaunchListed)
-    hipLaunchKernelGGL((listed_decode_kernel<G, E, kWavesPerWg, PD>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((listed_decode_kernel<G, E, kWavesPerWg>), grid, block, 0, st, a);
   else if (kind == kLaunchVerified)
-    hipLaunchKernelGGL((streamk_decode_kernel<G, E, kWavesPerWg, PD, kModeVerified>), grid,
+    hipLaunchKernelGGL((streamk_decode_kernel<G, E, kWavesPerWg, kModeVerified>), grid,
                        block, 0, st, a);
   else if (kind == kLaunchApprox)
-    hipLaunchKernelGGL((streamk_decode_kernel<G, E, kWavesPerWg, PD, kModeApprox>), grid,
+    hipLaunchKernelGGL((streamk_decode_kernel<G, E, kWavesPerWg, kModeApprox>), grid,
                        block, 0, st, a);
   else
-    hipLaunchKernelGGL((streamk_decode_kernel<G, E, kWavesPerWg, PD, kModeAll>), grid, block, 0,
+    hipLaunchKernelGGL((streamk_decode_kernel<G, E, kWavesPerWg, kModeAll>), grid, block, 0,
                        st, a);
 }
 
 // 16-token pages run engines with the tile shift compiled in (0).
 template <int G, int D>
-void launch_decode_gd(const DecodeArgs &a, int kind, dim3 grid, dim3 block, hipStream_t st) {
+void launch_decode_gd(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
   if (a.ts == 0 && a.tl == 4)
-    launch_decode_gdt<G, D, 0>(a, kind, grid, block, st);
+    launch_decode_gdt<G, D, 0>(a, kind, grid, st);
   else
-    launch_decode_gdt<G, D, -1>(a, kind, grid, block, st);
+    launch_decode_gdt<G, D, -1>(a, kind, grid, st);
 }
 
 template <int G>
-void launch_decode_g(const DecodeArgs &a, int kind, dim3 grid, dim3 block, hipStream_t st) {
+void launch_decode_g(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
   if (a.D == 32)
-    launch_decode_gd<G, 32>(a, kind, grid, block, st);
+    launch_decode_gd<G, 32>(a, kind, grid, st);
   else if (a.D == 64)
-    launch_decode_gd<G, 64>(a, kind, grid, block, st);
+    launch_decode_gd<G, 64>(a, kind, grid, st);
   else if (a.D == 256)
-    launch_decode_gd<G, 256>(a, kind, grid, block, st);
+    launch_decode_gd<G, 256>(a, kind, grid, st);
   else
-    launch_decode_gd<G, 128>(a, kind, grid, block, st);
+    launch_decode_gd<G, 128>(a, kind, grid, st);
 }
 
 // The reuse step's listed decode with the token append (D = 128, 16-token
 // pages).
 template <int G>
 void launch_append_g(const DecodeArgs &a, const AppendArgs &app, dim3 grid, hipStream_t st) {
-  hipLaunchKernelGGL((listed_append_kernel<G, MfmaEngine<G, 128, 0>, kWavesPerWg, 2>), grid,
+  hipLaunchKernelGGL((listed_append_kernel<G, MfmaEngine<G, 128, 0>, kWavesPerWg>), grid,
                      dim3(kWavesPerWg * kWave), 0, st, a, app);
 }
 
@@ -1605,15 +1651,15 @@ template <int G>
 void launch_spec_g(const DecodeArgs &a, const ScoreArgs &s, int score_gx, dim3 grid,
                    hipStream_t st) {
   if (a.ts == 0 && a.tl == 4)
-    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, 0>, kWavesPerWg, 2>), grid,
+    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, 0>, kWavesPerWg>), grid,
                        dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
   else
-    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, -1>, kWavesPerWg, 2>), grid,
+    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, -1>, kWavesPerWg>), grid,
                        dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
 }
 
 #define CVSA_DECODE_LAUNCHERS(PREFIX, GG)                                                    \
-  PREFIX template void launch_decode_g<GG>(const DecodeArgs &, int, dim3, dim3, hipStream_t); \
+  PREFIX template void launch_decode_g<GG>(const DecodeArgs &, int, dim3, hipStream_t); \
   PREFIX template void launch_spec_g<GG>(const DecodeArgs &, const ScoreArgs &, int, dim3,   \
                                          hipStream_t);                                         \
   PREFIX template void launch_append_g<GG>(const DecodeArgs &, const AppendArgs &, dim3,      \

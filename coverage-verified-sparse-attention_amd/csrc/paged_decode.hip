@@ -221,7 +221,7 @@ static void bind_workspace(DecodeArgs &a, void *workspace, size_t need) {
 static int enqueue_decode(const char *name, DecodeArgs a, int G, bool listed,
                           const DecodeLaunch &p, void *workspace, size_t need, hipStream_t st) {
   bind_workspace(a, workspace, need);
-  const dim3 grid(p.grid_x, p.grid_y), block(kWavesPerWg * kWave);
+  const dim3 grid(p.grid_x, p.grid_y);
   const int kind = !p.streamk ? kLaunchListed
                    : !listed   ? kLaunchAll
                    : a.alt_idx != nullptr ? kLaunchApprox
@@ -237,7 +237,7 @@ static int enqueue_decode(const char *name, DecodeArgs a, int G, bool listed,
     switch (min(kMaxGroup, G - off)) {
 #define CVSA_DEC_CASE(GG)                             \
   case GG:                                            \
-    launch_decode_g<GG>(a, kind, grid, block, st);    \
+    launch_decode_g<GG>(a, kind, grid, st);    \
     break;
       CVSA_DEC_CASE(1) CVSA_DEC_CASE(2) CVSA_DEC_CASE(3) CVSA_DEC_CASE(4)
       CVSA_DEC_CASE(5) CVSA_DEC_CASE(6) CVSA_DEC_CASE(7) CVSA_DEC_CASE(8)

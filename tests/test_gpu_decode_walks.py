@@ -1,0 +1,79 @@
+"""Decode walks at the edges of a wave's chunk of 64 tiles: a wave looks its
+tiles up 64 at a time, requests each tile while the one before it is used,
+and runs on from one chunk into the next.  Page counts around one tile per
+wave, one and two chunks, mixed over the heads of one launch, against a
+float32 restatement of the softmax over the listed tokens
+(cvsa/kernels/sparse_decode.py:76-124)."""
+import pytest
+import torch
+
+from cvsa import ops
+
+pytestmark = pytest.mark.gpu
+
+# Four waves share a workgroup's pages: 4 * 64 pages are one chunk each.
+COUNTS = (0, 1, 3, 4, 5, 8, 255, 256, 257, 260, 261, 511, 512, 513, 516, 520)
+
+
+def _reference(q, k, v, bt, pages, ctx, b, h, G, bs):
+    """(o, m, l, sum p |v|) of one KV head over the tokens of `pages`."""
+    tok = (pages[:, None] * bs + torch.arange(bs, device=q.device)).reshape(-1)
+    rows = bt[b, pages].long()
+    K = k[rows, :, h].reshape(-1, k.shape[3])[tok < ctx].float()
+    V = v[rows, :, h].reshape(-1, k.shape[3])[tok < ctx].float()
+    Q = q[b, h * G:(h + 1) * G].float()
+    s = (Q @ K.t().contiguous()) * k.shape[3] ** -0.5
+    m = s.amax(1)
+    p = torch.exp(s - m[:, None])
+    return p @ V, m, p.sum(1), p @ V.abs()
+
+
+@pytest.mark.parametrize("B,H,G,D,bs", [(64, 4, 4, 128, 16), (128, 2, 1, 64, 16),
+                                        (64, 4, 7, 128, 32), (64, 4, 2, 256, 16),
+                                        (32, 8, 8, 128, 8), (64, 4, 3, 32, 64)])
+def test_walks_across_chunks(gpu, B, H, G, D, bs):
+    """256 heads, so a listed head's pages all lie in one workgroup; the
+    listed decode, a verified launch with every other head rejected and the
+    dense decode."""
+    g = torch.Generator(device=gpu)
+    g.manual_seed(B + D + bs)
+    tiles = max(1, bs // 16)
+    W = -(-max(COUNTS) // tiles)
+    nb = 96  # pages share blocks: only the walk's order matters here
+    shape = (nb, bs, H, D)
+    k = torch.randn(shape, generator=g, device=gpu).to(torch.bfloat16)
+    v = torch.randn(shape, generator=g, device=gpu).to(torch.bfloat16)
+    q = torch.randn(B, H * G, D, generator=g, device=gpu).to(torch.bfloat16)
+    bt = torch.randint(nb, (B, W), generator=g, device=gpu, dtype=torch.int32)
+    ctx = torch.full((B,), W * bs, dtype=torch.int32, device=gpu)
+    ctx[1::3] -= bs // 2 + 1  # a partial last page
+    ctx[2] = max(1, bs // 2)
+    nv = (ctx + bs - 1) // bs
+    n = torch.tensor([-(-c // tiles) for c in COUNTS], device=gpu).repeat(B * H // 16)
+    n = torch.minimum(n[:B * H].view(B, H), nv[:, None]).to(torch.int32)
+    order = torch.rand(B, H, W, generator=g, device=gpu)
+    order = order.masked_fill(torch.arange(W, device=gpu) >= nv[:, None, None], 2.0)
+    idx = order.argsort(-1).to(torch.int32).contiguous()
+    acc = (torch.arange(B * H, device=gpu) % 2 == 0).view(B, H)
+    args = (q, k, v, bt)
+    listed = ops.sparse_decode_unnorm(*args, idx, n, ctx, H, G, bs)
+    _, ver = ops.verified_decode(*args, ctx, idx, n, acc, H, G, bs, return_state=True)
+    _, dense = ops.dense_decode(*args, ctx, H, G, bs, return_state=True)
+    cl, cn = ctx.tolist(), n.tolist()
+    for b in range(0, B, 3):
+        for h in range(H):
+            every = torch.arange(nv[b].item(), device=gpu)
+            sel = idx[b, h, :cn[b][h]].long()
+            full = _reference(q, k, v, bt, every, cl[b], b, h, G, bs)
+            part = _reference(q, k, v, bt, sel, cl[b], b, h, G, bs) if cn[b][h] else None
+            for got, want in ((listed, part), (ver, part if acc[b, h] else full),
+                              (dense, full)):
+                o, m, l = (t[b, h * G:(h + 1) * G] for t in got)
+                if want is None:  # no page: (0, -inf, 0)
+                    assert not o.any() and not l.any() and bool((m == -float("inf")).all())
+                    continue
+                # P is held to 16 mantissa bits and a score to ~1e-6 of |s| <= 8:
+                # each product is off by at most 2^-16 + 1e-5 of itself.
+                assert bool(((o - want[0]).abs() <= 4e-5 * want[3] + 1e-6).all()), (b, h)
+                assert torch.allclose(m, want[1], rtol=0, atol=2e-5), (b, h)
+                assert torch.allclose(l, want[2], rtol=4e-5), (b, h)
