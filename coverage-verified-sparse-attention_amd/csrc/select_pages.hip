@@ -14,9 +14,9 @@
 // scores (:198-208), coverage = exp(lse_sel - lse_all) and accept =
 // coverage >= tau compared in fp32 (:211-212).
 //
-// One 1024-thread workgroup per (b, kv-head); thread t owns the R
+// One workgroup of NT threads per (b, kv-head); thread t owns the R
 // consecutive pages [t*R, t*R + R).  The k-th largest score is found in two
-// steps: a 4096-bucket histogram over the row's finite value range [min, max]
+// steps: a histogram of 4 NT buckets over the row's finite value range [min, max]
 // (the bucket of a value is a non-decreasing function of it, so the k-th
 // largest lies in the bucket where the count from the top reaches k), then
 // one wave ranks the few scores of that bucket against each other.  Rows
@@ -55,15 +55,17 @@ __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
-// Bucket of a finite score in [vmin, vmin + kBuckets / inv]: a composition of
+// Bucket (of NB) of a finite score in [vmin, vmin + NB / inv]: a composition of
 // correctly rounded, monotone operations, so it never decreases as v grows,
 // and every evaluation gives the same bits (no fast-math in this library).
+template <int NB = kBuckets>
 __device__ __forceinline__ int value_bucket(float v, float vmin, float inv) {
-  return (int)fminf((v - vmin) * inv, (float)(kBuckets - 1));
+  return (int)fminf((v - vmin) * inv, (float)(NB - 1));
 }
 
 // Block-wide max of two keys and sum of one counter, one barrier.  `red`
 // holds 3 x kSelWaves words and is not reused by another reduction.
+template <int NW = kSelWaves>
 __device__ __forceinline__ void block_range(uint32_t &kmax, uint32_t &kneg, uint32_t &cnt,
                                             uint32_t (*red)[3]) {
   kmax = wave_max_u32(kmax);
@@ -80,7 +82,7 @@ __device__ __forceinline__ void block_range(uint32_t &kmax, uint32_t &kneg, uint
   kneg = red[0][1];
   cnt = red[0][2];
 #pragma unroll
-  for (int w = 1; w < kSelWaves; ++w) {
+  for (int w = 1; w < NW; ++w) {
     kmax = max(kmax, red[w][0]);
     kneg = max(kneg, red[w][1]);
     cnt += red[w][2];
@@ -93,6 +95,7 @@ __device__ __forceinline__ void stat_add(long long *p, long long v) {
 }
 
 // Exclusive prefix sum of one uint32 per thread over the block, plus total.
+template <int NW = kSelWaves>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *wsum,
                                                          uint32_t &total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -102,7 +105,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *w
   lds_barrier();
   uint32_t before = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < kSelWaves; ++w) {
+  for (int w = 0; w < NW; ++w) {
     const uint32_t s = wsum[w];
     before += (w < wave) ? s : 0u;
     tot += s;
@@ -112,6 +115,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *w
 }
 
 // Exclusive prefix sum of one uint64 per thread over the block, plus total.
+template <int NW = kSelWaves>
 __device__ __forceinline__ unsigned long long block_exclusive_scan_u64(
     unsigned long long v, unsigned long long *wsum64, unsigned long long &total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -126,7 +130,7 @@ __device__ __forceinline__ unsigned long long block_exclusive_scan_u64(
   lds_barrier();
   unsigned long long before = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < kSelWaves; ++w) {
+  for (int w = 0; w < NW; ++w) {
     const unsigned long long x = wsum64[w];
     before += (w < wave) ? x : 0ull;
     tot += x;
@@ -143,6 +147,7 @@ __device__ __forceinline__ float lse_from(float mx_floor, float sum) {
 
 // Max (first) and sum (second) of two values over the block; `red` holds
 // 2 x kSelWaves floats and is not reused by the other.
+template <int NW = kSelWaves>
 __device__ __forceinline__ void block_max2(float &a, float &b, float (*red)[2]) {
   a = wave_max_from_groups<1>(a);
   b = wave_max_from_groups<1>(b);
@@ -155,7 +160,7 @@ __device__ __forceinline__ void block_max2(float &a, float &b, float (*red)[2]) 
   a = red[0][0];
   b = red[0][1];
 #pragma unroll
-  for (int w = 1; w < kSelWaves; ++w) {
+  for (int w = 1; w < NW; ++w) {
     a = fmaxf(a, red[w][0]);
     b = fmaxf(b, red[w][1]);
   }
@@ -163,6 +168,7 @@ __device__ __forceinline__ void block_max2(float &a, float &b, float (*red)[2]) 
 
 // Sums of a and b and the max of c over the block in one barrier; `red`
 // holds 3 x kSelWaves floats and is not reused by another reduction.
+template <int NW = kSelWaves>
 __device__ __forceinline__ void block_sum2_max1(float &a, float &b, float &c, float (*red)[3]) {
   a = wave_sum_from_groups<1>(a);
   b = wave_sum_from_groups<1>(b);
@@ -178,13 +184,14 @@ __device__ __forceinline__ void block_sum2_max1(float &a, float &b, float &c, fl
   b = red[0][1];
   c = red[0][2];
 #pragma unroll
-  for (int w = 1; w < kSelWaves; ++w) {
+  for (int w = 1; w < NW; ++w) {
     a += red[w][0];
     b += red[w][1];
     c = fmaxf(c, red[w][2]);
   }
 }
 
+template <int NW = kSelWaves>
 __device__ __forceinline__ void block_sum1(float &a, float *red) {
   a = wave_sum_from_groups<1>(a);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -192,9 +199,10 @@ __device__ __forceinline__ void block_sum1(float &a, float *red) {
   lds_barrier();
   a = red[0];
 #pragma unroll
-  for (int w = 1; w < kSelWaves; ++w) a += red[w];
+  for (int w = 1; w < NW; ++w) a += red[w];
 }
 
+template <int NW = kSelWaves>
 __device__ __forceinline__ void block_sum2(float &a, float &b, float (*red)[2]) {
   a = wave_sum_from_groups<1>(a);
   b = wave_sum_from_groups<1>(b);
@@ -207,7 +215,7 @@ __device__ __forceinline__ void block_sum2(float &a, float &b, float (*red)[2]) 
   a = red[0][0];
   b = red[0][1];
 #pragma unroll
-  for (int w = 1; w < kSelWaves; ++w) {
+  for (int w = 1; w < NW; ++w) {
     a += red[w][0];
     b += red[w][1];
   }
@@ -218,15 +226,16 @@ __device__ __forceinline__ void block_sum2(float &a, float &b, float (*red)[2]) 
 // (behind an LDS barrier); returns the digit holding the krem-th largest of
 // them and krem minus the number of those keys with a higher digit.  Ends
 // with the histograms free for the next pass.
+template <int NT = kSelThreads>
 __device__ __forceinline__ void radix_digit(const uint32_t *hist_c, uint32_t *hist,
                                             uint32_t krem, uint32_t *s_digit, uint32_t *s_krem,
                                             uint32_t &digit, uint32_t &krem_out) {
   const int t = threadIdx.x, lane = t & 63;
-  if (t < 256) {
+  for (int i = t; i < 256; i += NT) {
     uint32_t c = 0;
 #pragma unroll
-    for (int j = 0; j < kHistCopies; ++j) c += hist_c[j * kHistStride + t];
-    hist[t] = c;
+    for (int j = 0; j < kHistCopies; ++j) c += hist_c[j * kHistStride + i];
+    hist[i] = c;
   }
   lds_barrier();
   if (t < 64) {
@@ -263,7 +272,7 @@ __device__ __forceinline__ void radix_digit(const uint32_t *hist_c, uint32_t *hi
 // into copy (lane % kHistCopies) of the histogram, rows padded by one word so
 // that the copies of a bin sit in different LDS banks: scores cluster in a
 // few leading digits, so lanes of one instruction often hit the same bin.
-template <int R, typename Alive>
+template <int R, int NT, typename Alive>
 __device__ __forceinline__ void radix_select(const float (&val)[R], Alive alive, uint32_t k,
                                              uint32_t *hist, uint32_t *hist_c,
                                              uint32_t *s_digit, uint32_t *s_krem,
@@ -274,7 +283,7 @@ __device__ __forceinline__ void radix_select(const float (&val)[R], Alive alive,
 #pragma unroll 1
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
-    for (int i = t; i < kHistCopies * kHistStride; i += kSelThreads) hist_c[i] = 0;
+    for (int i = t; i < kHistCopies * kHistStride; i += NT) hist_c[i] = 0;
     lds_barrier();
     uint32_t *my_hist = hist_c + (lane % kHistCopies) * kHistStride;
 #pragma unroll
@@ -284,7 +293,7 @@ __device__ __forceinline__ void radix_select(const float (&val)[R], Alive alive,
     }
     lds_barrier();
     uint32_t digit;
-    radix_digit(hist_c, hist, krem, s_digit, s_krem, digit, krem);
+    radix_digit<NT>(hist_c, hist, krem, s_digit, s_krem, digit, krem);
     prefix |= digit << shift;
     pmask |= 0xFFu << shift;
   }
@@ -298,6 +307,7 @@ __device__ __forceinline__ void radix_select(const float (&val)[R], Alive alive,
 // has nothing left to do); otherwise a fresh selection replaces it in place.
 // Counters: stats[0] accept-all checks, [1] rejections, [2] scoring steps,
 // [3] heads that passed the check.  All barriers here order LDS only.
+template <int NT = kSelThreads>
 __device__ __forceinline__ bool lazy_decision(
     const uint8_t *__restrict__ check_accept, int n_heads, int bh, int b, int width,
     int block_size, const int32_t *__restrict__ n_per_head,
@@ -328,7 +338,7 @@ __device__ __forceinline__ bool lazy_decision(
       }
       lds_barrier();
       int cnt = 0, bad = 0;
-      for (int i = t; i < n_heads; i += kSelThreads) {
+      for (int i = t; i < n_heads; i += NT) {
         const int v = check_accept[i] != 0;
         cnt += v;
         bad |= !v;
@@ -382,8 +392,8 @@ static_assert(kHistCopies * kHistStride >= kBuckets, "hist_c holds a second-leve
 // SEP: the selection ranks sel_scores while the coverage gate (and
 // scores_cache) use scores (CVSABackend._scoring_step, backend.py:723-727:
 // the Quest selector proposes, the exact scan verifies).
-template <int R, bool SEP, int MODE>
-__global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
+template <int NT, int R, bool SEP, int MODE>
+__global__ __launch_bounds__(NT) void select_topk_kernel(
     const float *__restrict__ scores, const float *__restrict__ sel_scores, int W, int H_kv,
     const int32_t *__restrict__ context_lens, int block_size, int budget, int width,
     float top_p, const int32_t *__restrict__ row_budgets,
@@ -394,22 +404,24 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     uint8_t *__restrict__ sel_map, int64_t map_stride,
     unsigned long long *__restrict__ keep_work, int exp_budget,
     int32_t *__restrict__ exp_indices) {
+  constexpr int kWaves = NT / kWave;
+  constexpr int NB = kBucketsPerThread * NT;  // value buckets
   __shared__ uint32_t hist[256];
   __shared__ uint32_t hist_c[kHistCopies * kHistStride];
-  __shared__ uint32_t hist_b[kBuckets];
+  __shared__ uint32_t hist_b[NB];
   __shared__ uint32_t s_cand[kRankCands];
-  __shared__ uint32_t wsum[kSelWaves];
-  __shared__ uint32_t red_rng[kSelWaves][3];
-  __shared__ float red_max[kSelWaves][2], red_sum[kSelWaves][2], red_s3[kSelWaves][3];
-  __shared__ float red_s1[kSelWaves];
+  __shared__ uint32_t wsum[kWaves];
+  __shared__ uint32_t red_rng[kWaves][3];
+  __shared__ float red_max[kWaves][2], red_sum[kWaves][2], red_s3[kWaves][3];
+  __shared__ float red_s1[kWaves];
   __shared__ uint32_t s_digit, s_krem, s_T, s_bucket, s_kb, s_nb, s_ncand;
   __shared__ int s_nok, s_nbad, s_acc;
   // Top-p only: softmax mass per value bucket (64-bit fixed point, so the
   // sums do not depend on the order of the atomic adds).
-  __shared__ unsigned long long mass_b[MODE == kTopP ? kBuckets : 1];
+  __shared__ unsigned long long mass_b[MODE == kTopP ? NB : 1];
   __shared__ unsigned long long s_candm[MODE == kTopP ? kRankCands : 1];
   __shared__ uint32_t s_candi[MODE == kTopP ? kRankCands : 1];
-  __shared__ unsigned long long wsum64[MODE == kTopP ? kSelWaves : 1];
+  __shared__ unsigned long long wsum64[MODE == kTopP ? kWaves : 1];
   __shared__ unsigned long long s_mass;
 
   const int bh = blockIdx.x;
@@ -432,7 +444,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
   // stores issued before them are not waited for.  (Scalar loads count
   // with LDS operations, so even a context-length load here would hold up
   // the check's barriers.)
-  if (lazy_decision(check_accept, n_heads, bh, b, width, block_size, n_per_head, context_lens,
+  if (lazy_decision<NT>(check_accept, n_heads, bh, b, width, block_size, n_per_head, context_lens,
                     accept_out, stats, count_gate, keep_flag, keep_work, s_nok, s_nbad))
     return;
 
@@ -483,7 +495,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
   // Range of the finite scores (as keys) and their count; +inf / NaN
   // entries are counted in the high half of `cnt`.  -inf (pages past the
   // context) lies below every finite score.
-  for (int i = t; i < kBuckets; i += kSelThreads) hist_b[i] = 0;
+  for (int i = t; i < NB; i += NT) hist_b[i] = 0;
   if (t == 0) s_ncand = 0;
   uint32_t kmax = 0, kneg = 0, cnt = 0;
   const auto finite = [&](int r) { return i0 + r < W && fabsf(val[r]) <= 3.402823466e38f; };
@@ -498,10 +510,10 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
       cnt += 1u << 16;
     }
   }
-  block_range(kmax, kneg, cnt, red_rng);
+  block_range<kWaves>(kmax, kneg, cnt, red_rng);
   const uint32_t kmin = ~kneg, n_fin = cnt & 0xFFFFu, n_odd = cnt >> 16;
   float vmin = 0.f, inv = 0.f;
-  const auto bucket = [&](int r) { return finite(r) ? value_bucket(val[r], vmin, inv) : -1; };
+  const auto bucket = [&](int r) { return finite(r) ? value_bucket<NB>(val[r], vmin, inv) : -1; };
 
   // Top-p budget: 1 + the number of pages, in descending score order, whose
   // inclusive cumulative softmax mass is below top_p, clamped to [3, W]
@@ -519,7 +531,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     unsigned long long m[kBucketsPerThread], lm = 0;
 #pragma unroll
     for (int j = 0; j < kBucketsPerThread; ++j) {
-      const int idx = kBuckets - 1 - (kBucketsPerThread * t + j);
+      const int idx = NB - 1 - (kBucketsPerThread * t + j);
       c[j] = cnts[idx];
       m[j] = ms[idx];
       lc += c[j];
@@ -528,12 +540,12 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     if (t == 0) s_bucket = 0xFFFFFFFFu;
     uint32_t ctot;
     unsigned long long mtot;
-    uint32_t cab = block_exclusive_scan(lc, wsum, ctot);
-    unsigned long long mab = base + block_exclusive_scan_u64(lm, wsum64, mtot);
+    uint32_t cab = block_exclusive_scan<kWaves>(lc, wsum, ctot);
+    unsigned long long mab = base + block_exclusive_scan_u64<kWaves>(lm, wsum64, mtot);
 #pragma unroll
     for (int j = 0; j < kBucketsPerThread; ++j) {
       if (mab < target && mab + m[j] >= target) {
-        s_bucket = (uint32_t)(kBuckets - 1 - (kBucketsPerThread * t + j));
+        s_bucket = (uint32_t)(NB - 1 - (kBucketsPerThread * t + j));
         s_kb = cab;
         s_nb = c[j];
         s_mass = mab;
@@ -554,7 +566,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     unsigned long long part = 0, total = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) part += mass(r);
-    (void)block_exclusive_scan_u64(part, wsum64, total);
+    (void)block_exclusive_scan_u64<kWaves>(part, wsum64, total);
     const unsigned long long target =
         (unsigned long long)ceil((double)top_p * (double)total);
     uint32_t before = 0;          // pages ranked above the range still to walk
@@ -562,11 +574,11 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     int lvl = 0, b1 = -1, b2 = -1;
     float vmin2 = 0.f, inv2 = 0.f;
     const float lo = key_value(kmin);
-    const float inv1 = (float)kBuckets / (M - lo);
+    const float inv1 = (float)NB / (M - lo);
     if (kmin != kmax && inv1 > 0.f && inv1 <= 3.402823466e38f) {
       vmin = lo;  // the buckets of the top-k below
       inv = inv1;
-      for (int i = t; i < kBuckets; i += kSelThreads) mass_b[i] = 0ull;
+      for (int i = t; i < NB; i += NT) mass_b[i] = 0ull;
       lds_barrier();
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -626,12 +638,12 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
           kn = max(kn, ~key);
         }
       }
-      block_range(kx, kn, cn, red_rng);
+      block_range<kWaves>(kx, kn, cn, red_rng);
       if (kx != ~kn) {
         vmin2 = key_value(~kn);
-        inv2 = (float)kBuckets / (key_value(kx) - vmin2);
+        inv2 = (float)NB / (key_value(kx) - vmin2);
         if (inv2 > 0.f && inv2 <= 3.402823466e38f) {
-          for (int i = t; i < kBuckets; i += kSelThreads) {
+          for (int i = t; i < NB; i += NT) {
             hist_c[i] = 0u;
             mass_b[i] = 0ull;
           }
@@ -639,7 +651,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             if (bucket(r) == b1) {
-              const int bk = value_bucket(val[r], vmin2, inv2);
+              const int bk = value_bucket<NB>(val[r], vmin2, inv2);
               atomicAdd(&hist_c[bk], 1u);
               atomicAdd(&mass_b[bk], mass(r));
             }
@@ -660,13 +672,13 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
       if (!finite(r)) return false;
       if (lvl == 0) return true;
       if (bucket(r) != b1) return false;
-      return lvl == 1 || value_bucket(val[r], vmin2, inv2) == b2;
+      return lvl == 1 || value_bucket<NB>(val[r], vmin2, inv2) == b2;
     };
     unsigned long long mine = 0, tot = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r)
       if (in_range(r)) mine += mass(r);
-    unsigned long long run = base + block_exclusive_scan_u64(mine, wsum64, tot);
+    unsigned long long run = base + block_exclusive_scan_u64<kWaves>(mine, wsum64, tot);
     uint32_t lt = 0, lt_total = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -675,7 +687,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
         lt += run < target ? 1u : 0u;
       }
     }
-    (void)block_exclusive_scan(lt, wsum, lt_total);
+    (void)block_exclusive_scan<kWaves>(lt, wsum, lt_total);
     return min(max((int)(before + lt_total + 1), 3), W);
   };
 
@@ -705,7 +717,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
       plan = 0;
     } else if (n_odd == 0) {
       vmin = key_value(kmin);
-      inv = (float)kBuckets / (key_value(kmax) - vmin);
+      inv = (float)NB / (key_value(kmax) - vmin);
       // Otherwise max - min overflows.
       if (inv > 0.f && inv <= 3.402823466e38f) {
         if (!hist_ready) {
@@ -717,20 +729,20 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
           hist_ready = true;
         }
         lds_barrier();
-        // Thread t holds buckets kBuckets-1-(4t+j), j = 0..3: the exclusive
+        // Thread t holds buckets NB-1-(4t+j), j = 0..3: the exclusive
         // scan over threads counts the scores in higher buckets.
         uint32_t c[kBucketsPerThread], local = 0;
 #pragma unroll
         for (int j = 0; j < kBucketsPerThread; ++j) {
-          c[j] = hist_b[kBuckets - 1 - (kBucketsPerThread * t + j)];
+          c[j] = hist_b[NB - 1 - (kBucketsPerThread * t + j)];
           local += c[j];
         }
         uint32_t total_b;
-        uint32_t above = block_exclusive_scan(local, wsum, total_b);
+        uint32_t above = block_exclusive_scan<kWaves>(local, wsum, total_b);
 #pragma unroll
         for (int j = 0; j < kBucketsPerThread; ++j) {
           if (above < (uint32_t)kk && above + c[j] >= (uint32_t)kk) {
-            s_bucket = (uint32_t)(kBuckets - 1 - (kBucketsPerThread * t + j));
+            s_bucket = (uint32_t)(NB - 1 - (kBucketsPerThread * t + j));
             s_kb = (uint32_t)kk - above;
             s_nb = c[j];
           }
@@ -738,7 +750,8 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
         }
         lds_barrier();
         bstar = (int)s_bucket;
-        const uint32_t kb = s_kb, nb = s_nb;
+        const uint32_t kb = s_kb;
+        const uint32_t nb = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_nb);
         // The buckets are recomputed below rather than kept live across the
         // scan (same operands, same bits).
         asm volatile("" : "+v"(vmin), "+v"(inv));
@@ -751,8 +764,8 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
           if (t < kWave) {
             const uint32_t mine = t < (int)nb ? s_cand[t] : 0u;
             uint32_t gt = 0, eq = 0;
-            for (uint32_t j = 0; j < nb; ++j) {
-              const uint32_t o = s_cand[j];
+            for (uint32_t j = 0; j < nb; ++j) {  // nb is the same in every lane
+              const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j);
               gt += o > mine;
               eq += o == mine;
             }
@@ -774,7 +787,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     }
     if (plan != 0) {
       const auto alive = [&](int r) { return i0 + r < W && (plan == 1 || bucket(r) == bstar); };
-      radix_select<R>(val, alive, k_radix, hist, hist_c, &s_digit, &s_krem, T, krem);
+      radix_select<R, NT>(val, alive, k_radix, hist, hist_c, &s_digit, &s_krem, T, krem);
     }
   };
 
@@ -793,7 +806,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
       }
     }
     uint32_t total;
-    const uint32_t excl = block_exclusive_scan(gt | (eq << 16), wsum, total);
+    const uint32_t excl = block_exclusive_scan<kWaves>(gt | (eq << 16), wsum, total);
     const uint32_t gt_before = excl & 0xFFFFu, eq_before = excl >> 16;
     uint32_t eq_seen = eq_before;
     uint32_t pos = gt_before + min(eq_before, krem);
@@ -859,7 +872,7 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
       mx = fmaxf(mx, gate(r));
       if (counted[r]) ms = fmaxf(ms, gate(r));
     }
-    block_max2(mx, ms, red_max);
+    block_max2<kWaves>(mx, ms, red_max);
   }
   const float m_all = fmaxf(mx, -1e20f);
   // Padding lanes of the reference's power-of-two selection block carry
@@ -877,17 +890,17 @@ __global__ __launch_bounds__(kSelThreads) void select_topk_kernel(
     }
   }
   if (fast_max) {
-    block_sum2_max1(se, ss, ms_true, red_s3);
+    block_sum2_max1<kWaves>(se, ss, ms_true, red_s3);
     if (ms_true != ms) {  // uniform; the counted pages miss the row's maximum
       m_sel = n_sel < msel_block ? fmaxf(ms_true, -1e20f) : ms_true;
       ss = 0.f;
 #pragma unroll
       for (int r = 0; r < R; ++r)
         if (counted[r]) ss += fast_exp(gate(r) - m_sel);
-      block_sum1(ss, red_s1);
+      block_sum1<kWaves>(ss, red_s1);
     }
   } else {
-    block_sum2(se, ss, red_sum);
+    block_sum2<kWaves>(se, ss, red_sum);
   }
   if (t == 0) {
     const float cov = expf(lse_from(m_sel, ss) - lse_from(m_all, se));
@@ -1146,7 +1159,7 @@ __device__ __forceinline__ void wide_threshold(const float *__restrict__ row, in
 #pragma unroll
   for (int r = 0; r < RC; ++r) cv[r] = L.cand[min(t + r * kSelThreads, kWideCands - 1)];
   const auto alive = [&](int r) { return (uint32_t)(t + r * kSelThreads) < nb; };
-  radix_select<RC>(cv, alive, kb, L.hist, L.hist_c, &L.digit, &L.krem, T, krem);
+  radix_select<RC, kSelThreads>(cv, alive, kb, L.hist, L.hist_c, &L.digit, &L.krem, T, krem);
 }
 
 // Ascending compaction of a wide row's selection (T, krem) into out_row
@@ -1597,12 +1610,19 @@ __global__ __launch_bounds__(kSelThreads) void check_coverage_wide_kernel(
   }
 }
 
-static int keys_per_thread(int n) {
+static int keys_per_thread(int n, int threads = kSelThreads) {
   int r = 1;
-  while (r * kSelThreads < n) r <<= 1;
+  while (r * threads < n) r <<= 1;
   return r;
 }
 
+// Threads of the workgroup that selects from a row of W pages: 256 up to 1024
+// pages (its block-wide steps cross 4 waves instead of 16: 5.4 against 6.7 us
+// at 512 pages, 6.1-6.4 against 6.6-6.9 at 513-1024; select + gate, 8 to 256
+// rows), 1024 above (7.2 against 8.0-8.3 us at 1500-2047 pages, 9.2 against
+// 12.6 at 4096).  Top-p keeps 1024, whose 4096 buckets bound how finely its
+// second level resolves the crossing.
+static int select_threads(int W) { return W <= 1024 ? 256 : kSelThreads; }
 
 static int launch_select(const char *name, const float *page_scores, const float *sel_scores,
                          int32_t B, int32_t H_kv,
@@ -1642,7 +1662,6 @@ static int launch_select(const char *name, const float *page_scores, const float
                "%s: an expanded selection needs the uniform budget, the gate and an expanded "
                "budget in [1, W=%d] (got %d)",
                name, W, exp_budget);
-  const int R = keys_per_thread(W);
   const dim3 grid(B * H_kv);
   hipStream_t st = (hipStream_t)stream;
   long long *st64 = reinterpret_cast<long long *>(stats);
@@ -1675,32 +1694,44 @@ static int launch_select(const char *name, const float *page_scores, const float
     }
     return cvsa_host::check_launch(name);
   }
-  switch (R) {
-#define CVSA_SEL_LAUNCH(RR, SEP, MODE)                                                      \
-  hipLaunchKernelGGL((select_topk_kernel<RR, SEP, MODE>), grid, dim3(kSelThreads), 0, st,   \
+#define CVSA_SEL_LAUNCH(NT, RR, SEP, MODE)                                                   \
+  hipLaunchKernelGGL((select_topk_kernel<NT, RR, SEP, MODE>), grid, dim3(NT), 0, st,         \
                      page_scores, sel_scores, W, H_kv, context_lens, block_size, budget,    \
                      width, top_p, row_budgets, page_indices, n_per_head, tau, accept_out,  \
                      coverage_out, check_accept, B * H_kv, scores_cache, st64, count_gate,    \
                      keep_flag, sel_map, map_stride,                                         \
                      reinterpret_cast<unsigned long long *>(keep_work), exp_budget, exp_indices)
-#define CVSA_SEL_MODES(RR, SEP)                                    \
-  if (mode == kTopP) CVSA_SEL_LAUNCH(RR, SEP, kTopP);              \
-  else if (mode == kTable) CVSA_SEL_LAUNCH(RR, SEP, kTable);       \
-  else CVSA_SEL_LAUNCH(RR, SEP, kUniform);
-#define CVSA_SEL_CASE(RR)                                       \
-  case RR:                                                      \
+#define CVSA_SEL_MODES(NT, RR, SEP)                                \
+  if (mode == kTable) CVSA_SEL_LAUNCH(NT, RR, SEP, kTable);        \
+  else CVSA_SEL_LAUNCH(NT, RR, SEP, kUniform);
+#define CVSA_SEL_CASE(NT, RR)                                   \
+  case (NT) * 64 + RR:                                          \
     if (sel_scores != nullptr) {                                \
-      CVSA_SEL_MODES(RR, true)                                  \
+      CVSA_SEL_MODES(NT, RR, true)                              \
     } else {                                                    \
-      CVSA_SEL_MODES(RR, false)                                 \
+      CVSA_SEL_MODES(NT, RR, false)                             \
     }                                                           \
     break;
-    CVSA_SEL_CASE(1)
-    CVSA_SEL_CASE(2)
-    CVSA_SEL_CASE(4)
-    CVSA_SEL_CASE(8)
-    CVSA_SEL_CASE(16)
-    CVSA_SEL_CASE(32)
+#define CVSA_TOPP_CASE(RR)                                                              \
+  case RR:                                                                              \
+    if (sel_scores != nullptr) CVSA_SEL_LAUNCH(kSelThreads, RR, true, kTopP);           \
+    else CVSA_SEL_LAUNCH(kSelThreads, RR, false, kTopP);                                \
+    break;
+  if (mode == kTopP) {
+    switch (keys_per_thread(W, kSelThreads)) {
+      CVSA_TOPP_CASE(1) CVSA_TOPP_CASE(2) CVSA_TOPP_CASE(4)
+      CVSA_TOPP_CASE(8) CVSA_TOPP_CASE(16) CVSA_TOPP_CASE(32)
+      default:
+        return cvsa_host::fail(CVSA_ERR_UNSUPPORTED, "%s: W=%d too large", name, W);
+    }
+    return cvsa_host::check_launch(name);
+  }
+  const int nt = select_threads(W);
+  switch (nt * 64 + keys_per_thread(W, nt)) {
+    CVSA_SEL_CASE(256, 1) CVSA_SEL_CASE(256, 2) CVSA_SEL_CASE(256, 4)
+    CVSA_SEL_CASE(1024, 2) CVSA_SEL_CASE(1024, 4) CVSA_SEL_CASE(1024, 8)
+    CVSA_SEL_CASE(1024, 16) CVSA_SEL_CASE(1024, 32)
+#undef CVSA_TOPP_CASE
 #undef CVSA_SEL_CASE
 #undef CVSA_SEL_MODES
 #undef CVSA_SEL_LAUNCH
