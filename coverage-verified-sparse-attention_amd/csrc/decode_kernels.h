@@ -275,7 +275,7 @@ __device__ __forceinline__ int approx_booked_pages(const DecodeArgs &a, int bh, 
 // Stream-K partition.  The heads' page walks are concatenated (head-major)
 // into one list of T pages and cut into n_wg equal ranges; workgroup w owns
 // pages [start(w), start(w + 1)), start(w) = floor(w * T / n_wg).  n_wg is the
-// launch size, reduced so that a workgroup gets at least kMinPagesPerWg
+// launch size, reduced so that a workgroup gets at least kMinPagesPerSkWg
 // pages.  T < 2^31 and n_wg <= kMaxSplits, so every quantity is computed in
 // 32 bits (64-bit division is a long instruction sequence on the GPU).
 constexpr int kMaxHeads = 4096;  // B * H_kv of one launch
@@ -291,11 +291,16 @@ constexpr int kMergeGroup = 16;
 constexpr int kTwoLevelMin = 48;
 constexpr int kGroupCounters = 2 * 256;  // 2 x the largest stream-K grid
 constexpr int kMinPagesPerWg = kMinPagesPerWave * kWavesPerWg;
+// A stream-K workgroup takes at least this many pages, so a short launch has
+// fewer partials to hand off (a scoring step at B = 1, 8K, five of eight heads
+// recovered, 2944 pages: 8 pages per workgroup 29.2 us, 16 26.4, 24 30.4,
+// 32 28.0).
+constexpr int kMinPagesPerSkWg = 2 * kMinPagesPerWg;
 
 struct Partition {
   int T, n, q, r;  // pages, workgroups, T / n, T % n
   __device__ __forceinline__ Partition(int T_, int grid) : T(T_) {
-    n = max(1, min(grid, (T + kMinPagesPerWg - 1) / kMinPagesPerWg));
+    n = max(1, min(grid, (T + kMinPagesPerSkWg - 1) / kMinPagesPerSkWg));
     q = T / n;
     r = T - q * n;
   }
@@ -922,7 +927,8 @@ __device__ __forceinline__ void segment_epilogue(const DecodeArgs &a, const Part
                                                  WalkLds<G, Engine, NW> &lds) {
   constexpr int D = Engine::kD;
   constexpr int NT = NW * kWave;
-  constexpr int KMAX = TWO ? 8 : 16;
+  // Chunks past one per thread (G D > 4 NT) are merged in several passes.
+  constexpr int KMAX = TWO || G * D > 4 * NT ? 8 : 16;
   auto &s_m = lds.m;
   auto &s_l = lds.l;
   auto &s_last = lds.last;
@@ -1304,7 +1310,10 @@ void score_spec_kernel(const DecodeArgs a, const ScoreArgs s, int score_gx) {
 }
 
 // Every workgroup first computes the pages each head walks and their prefix
-// (the same partition in every workgroup), then walks the segments of its
+// (the same partition in every workgroup; the heads' counts and flags are
+// requested together, and nothing is walked on a guess: a mixed launch, whose
+// rejected heads walk other numbers of pages, would throw the guess away
+// along with 8 MiB of requests), then walks the segments of its
 // range: (head h, pages s0..s1 of h's walk).  A segment that is a whole head
 // writes the outputs; otherwise it stores a partial (o, m, l) in row w + h of
 // the partial buffer (unique: a later workgroup never starts at an earlier
@@ -1319,7 +1328,7 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
 
   __shared__ WalkLds<G, Engine, NW> L;
   __shared__ int s_wsum[NW];
-  __shared__ int s_odd[NW];               // a head of the wave's pass walks != max_sel pages
+  __shared__ int s_flags[NW];
   __shared__ int s_start[kMaxHeads + 1];  // exclusive prefix of pages per head
   __shared__ uint8_t s_listed[kMaxHeads];  // kWalk* of each head
   const int lane = threadIdx.x & 63;
@@ -1330,13 +1339,34 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
   const int ts = Engine::tshift(a);
   const int tl = Engine::tlog(a);
 
+  // Tiles per head, scanned into their exclusive prefix in s_start, one head
+  // per thread and pass of NT heads (loads issued without a branch, index
+  // clamped); T their sum.
+  int walk0 = kWalkAll, c0 = 0, T = 0;  // c0, walk0: head threadIdx.x
+  auto scan_pass = [&](int hh, int c, int walk) {
+    const int incl = (int)wave_incl_scan_u32((uint32_t)c);
+    if (lane == kWave - 1) s_wsum[wave] = incl;
+    lds_barrier();
+    int excl = incl - c, total = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      if (i < wave) excl += s_wsum[i];
+      total += s_wsum[i];
+    }
+    if (hh < heads) {
+      s_start[hh] = T + excl;
+      s_listed[hh] = (uint8_t)walk;
+    }
+    T += total;
+  };
+
   // Verified launches whose heads are all accepted (a lazy check that keeps
   // its selection, or a scoring step whose gate passes everywhere) run the
   // listed decode's static partition: workgroup w takes split w % n_splits
   // of head w / n_splits, exactly as listed_decode_kernel, so the outputs
   // are bit for bit those of the listed decode.  Its first page-list
-  // entries are requested together with the accept flags and spec_state,
-  // their block-table entries once the launch is known to walk.  When the
+  // entries are requested together with the heads' counts and flags and
+  // spec_state, their block-table entries once the launch is known to walk.  When the
   // check kept its selection (spec_state[0], written by the check's
   // select-or-keep) and a speculative listed decode of that selection
   // already wrote the outputs (spec_state[1]), there is nothing left: the
@@ -1348,21 +1378,29 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
     const int split = w % max(a.n_splits, 1);
     const int bh = min(w / max(a.n_splits, 1), heads - 1);
     const int lp = listed_first_entry<NW>(a, split, bh, wave, lane, Engine::tshift(a));
-    int spec_done = 0;
-    if (a.spec_state != nullptr)
-      spec_done = __builtin_amdgcn_readfirstlane(a.spec_state[0] == 1 && a.spec_state[1] == 1);
-    if (spec_done != 0) return;  // uniform; every head was accepted (kept)
-    int rejected = 0, accepted = 0;
-    for (int i = threadIdx.x; i < heads; i += NT) {
-      rejected |= a.accept[i] == 0;
-      accepted |= a.accept[i] != 0;
-    }
-    rejected = __syncthreads_or(rejected);
-    accepted = __syncthreads_or(accepted);
-    if (rejected == 0) {  // uniform
+    const bool has_spec = a.spec_state != nullptr;
+    const int spec_keep = has_spec ? a.spec_state[0] : 0, spec_ran = has_spec ? a.spec_state[1] : 0;
+    const bool acc0 = a.accept[min((int)threadIdx.x, heads - 1)] != 0;
+    if (__builtin_amdgcn_readfirstlane(spec_keep == 1 && spec_ran == 1) != 0)
+      return;  // uniform; every head was accepted (kept)
+    c0 = head_pages<MODE>(a, min((int)threadIdx.x, heads - 1), walk0, ts, tl);
+    // Whether some head is rejected, and some accepted: one barrier.
+    enum { kSomeRejected = 1, kSomeAccepted = 2 };
+    int f = acc0 ? kSomeAccepted : kSomeRejected;
+    for (int i = threadIdx.x + NT; i < heads; i += NT)
+      f |= a.accept[i] != 0 ? kSomeAccepted : kSomeRejected;
+    f = (__ballot(f & kSomeRejected) != 0 ? kSomeRejected : 0) |
+        (__ballot(f & kSomeAccepted) != 0 ? kSomeAccepted : 0);
+    if (lane == 0) s_flags[wave] = f;
+    lds_barrier();
+    int flags = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) flags |= s_flags[i];
+    flags = __builtin_amdgcn_readfirstlane(flags);
+    if ((flags & kSomeRejected) == 0) {  // uniform
       if (w < n_listed)
         listed_walk<G, Engine, NW>(a, split, bh, lp,
-                                       listed_first_block(a, bh, lp, Engine::tshift(a)), L);
+                                   listed_first_block(a, bh, lp, Engine::tshift(a)), L);
       return;
     }
     // Every head rejected (exact recovery: each attends all its valid
@@ -1370,10 +1408,9 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
     // decode of the lazy check (spec_state[1] == 2) already wrote with the
     // same bits; then only its effective-budget counters are booked.  The
     // next check of the layer is told to speculate that way again.
-    if (MODE == kModeVerified && accepted == 0) {  // uniform
-      const bool dense_done =
-          a.spec_state != nullptr && __builtin_amdgcn_readfirstlane(a.spec_state[1]) == 2;
-      if (w == 0 && threadIdx.x == 0 && a.spec_state != nullptr) a.spec_state[0] = 2;
+    if (MODE == kModeVerified && (flags & kSomeAccepted) == 0) {  // uniform
+      const bool dense_done = __builtin_amdgcn_readfirstlane(spec_ran) == 2;
+      if (w == 0 && threadIdx.x == 0 && has_spec) a.spec_state[0] = 2;
       if (dense_done) {
         if (w == 0 && a.work != nullptr) {
           for (int i = threadIdx.x; i < heads; i += NT) {
@@ -1391,133 +1428,22 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
       listed_walk<G, Engine, NW, false, false, true>(a, isplit, ibh, ilp, iphys, L);
       return;
     }
+  } else {
+    c0 = head_pages<MODE>(a, min((int)threadIdx.x, heads - 1), walk0, ts, tl);
   }
-
-  // Speculative page lookups for the common case in which every head walks
-  // max_sel listed pages: the range start is then known without the scan.
-  // The first page-list entries, the head's context length and q and the
-  // head counts of the scan are requested at entry, the pages' block-table
-  // entries as soon as the page-list entries arrive, and the first tile of
-  // K/V before the scan: two memory round trips fewer before the first
-  // K/V load.  Used only if the scan confirms the case.  The loads are
-  // issued without branches (indices clamped; a WG without a speculated
-  // range reads harmless in-bounds entries and discards them), so the
-  // compiler never has to drain them at a join.
-  Engine eng;
-  const int max_sel_t = a.max_sel << ts;  // tiles of a full selection
-  const int T_spec = heads * max_sel_t;
-  const Partition spec_part(T_spec, a.sk_grid);
-  int spec_lp = 0, spec_phys = 0, h_spec = -1, r_spec = 0, ctx_spec = 0, g1_spec = 0;
-  int b_spec = 0, h_c = 0;  // clamped speculated head and its sequence
-  if constexpr (MODE != kModeAll) {
-    const int ms = max(max_sel_t, 1);
-    const int wc = min(w, spec_part.n - 1);
-    const int g0 = spec_part.start(wc);
-    g1_spec = spec_part.start(wc + 1);
-    const int hs = min(g0 / ms, heads - 1);
-    r_spec = g0 - hs * ms;
-    h_c = hs;
-    b_spec = hs / a.H_kv;
-    const int rs = max(0, min(r_spec + wave + NW * lane, max_sel_t - 1));
-    const int32_t *src =
-        a.max_sel > 0 ? a.page_idx + (int64_t)hs * a.idx_stride + (rs >> ts) : a.block_tables;
-    const int lp0 = *src;
-    spec_lp = ts == 0 ? lp0 : lp0 >= 0 && lp0 < a.W ? (lp0 << ts) | (rs & ((1 << ts) - 1)) : -1;
-    ctx_spec = __builtin_amdgcn_readfirstlane(a.ctx_lens[b_spec]);
-    eng.init(a, b_spec, hs - b_spec * a.H_kv, lane);
-    if (a.max_sel > 0 && w < spec_part.n) h_spec = hs;
+  scan_pass(threadIdx.x, (int)threadIdx.x < heads ? c0 : 0, walk0);
+  for (int base = NT; base < heads; base += NT) {  // uniform
+    lds_barrier();  // s_wsum is rewritten
+    const int hh = base + threadIdx.x;
+    int walk = kWalkAll;
+    const int c = head_pages<MODE>(a, min(hh, heads - 1), walk, ts, tl);
+    scan_pass(hh, hh < heads ? c : 0, walk);
   }
-
-  // Pages per head, one head per thread and pass of NT heads (loads issued
-  // without a branch, index clamped), scanned into their exclusive prefix
-  // in s_start.
-  auto wave_incl_scan = [&](int c) { return (int)wave_incl_scan_u32((uint32_t)c); };
-  // A head walking its expanded selection never takes the speculated
-  // partition, whose first pages come from page_indices.
-  int l_first = kWalkAll;
-  int c_first = head_pages<MODE>(a, min((int)threadIdx.x, heads - 1), l_first, ts, tl);
-  if constexpr (MODE != kModeAll)
-    spec_phys = tile_block(a, b_spec, spec_lp, ts);
-  if ((int)threadIdx.x >= heads) c_first = 0;
-  const int incl_first = wave_incl_scan(c_first);
-  if (lane == kWave - 1) s_wsum[wave] = incl_first;
-  const bool odd_first =
-      __ballot((int)threadIdx.x < heads && (c_first != max_sel_t || l_first == kWalkAlt)) != 0;
-  if (lane == 0) s_odd[wave] = odd_first ? 1 : 0;
-
-  // Tiles c0 .. of a wave's part of a segment (its tiles s0 + wave + NW j,
-  // j < npw), one per lane; `spec` takes the speculative entries.
-  auto lookup = [&](int s0, int c0, int npw, bool listed, const int32_t *idx_row, int b,
-                    bool spec) {
-    const int r = s0 + wave + NW * min(c0 + lane, max(npw - 1, 0));
-    int lp = r, phys = 0;
-    if (spec) {
-      lp = spec_lp;
-      phys = spec_phys;
-    } else if (npw > 0) {
-      if (listed) lp = listed_tile(a, idx_row, r, ts);
-      phys = tile_block(a, b, lp, ts);
-    }
-    TileChunk c;
-    if (c0 + lane < npw && lp >= 0 && lp < (a.W << ts) && phys >= 0 &&
-        phys < (a.num_blocks << ts)) {
-      c.phys = phys;
-      c.lt = lp;
-    }
-    return c;
-  };
-
-  // First tile of the speculated segment (a WG without one reads nothing).
-  TileChunk first;
-  if constexpr (MODE != kModeAll) {
-    const int s1 = min(g1_spec, (h_c + 1) * max_sel_t) - h_c * max_sel_t;
-    const int npw = h_spec >= 0 ? max(0, (s1 - r_spec - wave + NW - 1) / NW) : 0;
-    first = lookup(r_spec, 0, npw, true, nullptr, b_spec, true);
-    start_walk<Engine>(a, eng, first);
-  }
-  // Pass 0 (peeled: a loop header here makes the compiler wait for the
-  // speculative loads), then the passes of launches with more than NT heads.
-  int uneven = 0;  // some head walks a number of pages other than max_sel
-  auto finish_pass = [&](int hh, int c, int incl, int lst, int &carry) {
-    lds_barrier();
-    int excl = incl - c, total = 0;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      if (i < wave) excl += s_wsum[i];
-      total += s_wsum[i];
-      uneven |= s_odd[i];
-    }
-    if (hh < heads) {
-      s_start[hh] = carry + excl;
-      s_listed[hh] = (uint8_t)lst;
-    }
-    carry += total;
-    lds_barrier();  // s_wsum is rewritten by the next pass
-  };
-  int carry = 0;
-  finish_pass(threadIdx.x, c_first, incl_first, l_first, carry);
-  if (heads > NT) {  // uniform
-    for (int base = NT; base < heads; base += NT) {
-      const int hh = base + threadIdx.x;
-      int lst = kWalkAll;
-      int c = head_pages<MODE>(a, min(hh, heads - 1), lst, ts, tl);
-      if (hh >= heads) c = 0;
-      const int incl = wave_incl_scan(c);
-      if (lane == kWave - 1) s_wsum[wave] = incl;
-      const bool odd = __ballot(hh < heads && (c != max_sel_t || lst == kWalkAlt)) != 0;
-      if (lane == 0) s_odd[wave] = odd ? 1 : 0;
-      finish_pass(hh, c, incl, lst, carry);
-    }
-  }
-  int T = carry;
   if (threadIdx.x == 0) s_start[heads] = T;
-  lds_barrier();
+  lds_barrier();  // s_start and s_listed
   T = __builtin_amdgcn_readfirstlane(T);
 
-  // Every head walks max_sel pages (a matching total is not enough: one
-  // head's extra pages can make up for another's missing ones).
-  const bool spec_ok = uneven == 0 && T == T_spec && h_spec >= 0;
-  const Partition part = spec_ok ? spec_part : Partition(max(T, 1), a.sk_grid);
+  const Partition part(max(T, 1), a.sk_grid);
   const int n_wg = T > 0 ? part.n : a.sk_grid;
   if (w >= n_wg) return;  // uniform
 
@@ -1537,17 +1463,16 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
   const int g0 = part.start(w);
   const int g1 = part.start(w + 1);
   // First head of the range: the last head that starts at or before g0 (it
-  // holds page g0, so it is not empty).
-  int lo = h_spec;
-  if (!spec_ok) {
-    lo = 0;
-    int hi = heads - 1;
-    while (lo < hi) {  // uniform binary search
-      const int mid = (lo + hi + 1) >> 1;
-      if (s_start[mid] <= g0) lo = mid;
-      else hi = mid - 1;
-    }
-  }
+  // holds tile g0, so it is not empty), a wave's worth of starts per read:
+  // every `step`-th head, then the heads of one step.
+  static_assert(kMaxHeads <= kWave * kWave, "two reads find the head");
+  const int step = (heads + kWave - 1) / kWave;
+  auto starts_at_or_before = [&](int h0, int each, int end) {
+    const int h = h0 + lane * each;
+    return __popcll(__ballot(h < end && s_start[min(h, heads)] <= g0));
+  };
+  int lo = (starts_at_or_before(0, step, heads) - 1) * step;
+  if (step > 1) lo += starts_at_or_before(lo, 1, min(lo + step, heads)) - 1;
   const PartBuf pb(a.part, a.part_bytes);
 
   for (int h = lo; h < heads; ++h) {
@@ -1560,23 +1485,32 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
     const int hk = h - b * a.H_kv;
     const int walk = s_listed[h];
     const bool listed = walk != kWalkAll;
-    const bool on_spec = h == h_spec;  // eng, ctx_spec already belong to this head
-    const int ctx = on_spec ? ctx_spec : __builtin_amdgcn_readfirstlane(a.ctx_lens[b]);
+    const int ctx = __builtin_amdgcn_readfirstlane(a.ctx_lens[b]);
     const int32_t *idx_row = MODE == kModeApprox && walk == kWalkAlt
                                  ? a.alt_idx + (int64_t)h * a.alt_stride
                                  : a.page_idx + (int64_t)h * a.idx_stride;
-    const bool use_spec = spec_ok && on_spec && s0 == r_spec && walk == kWalkListed;
-
-    if (!on_spec || h != lo) eng.init(a, b, hk, lane);
     const int npw = max(0, (s1 - s0 - wave + NW - 1) / NW);
-    if (!use_spec) {  // else the speculated first tile is already in flight
-      first = lookup(s0, 0, npw, listed, idx_row, b, false);
-      start_walk<Engine>(a, eng, first);
-    }
+    // Tiles e0 .. of the wave's part (tiles s0 + wave + NW e), one per lane.
+    auto lookup = [&](int e0) {
+      const int r = s0 + wave + NW * min(e0 + lane, max(npw - 1, 0));
+      const int lt = listed ? listed_tile(a, idx_row, r, ts) : r;
+      const int phys = tile_block(a, b, lt, ts);
+      TileChunk c;
+      if (e0 + lane < npw && lt >= 0 && lt < (a.W << ts) && phys >= 0 &&
+          phys < (a.num_blocks << ts)) {
+        c.phys = phys;
+        c.lt = lt;
+      }
+      return c;
+    };
+    TileChunk first;
+    if (npw > 0) first = lookup(0);
+    Engine eng;
+    eng.init(a, b, hk, lane);
+    start_walk<Engine>(a, eng, first);
     walk_tiles<Engine, false, false>(
-        a, eng, npw, ctx, first,
-        [&](int c0) { return lookup(s0, c0, npw, listed, idx_row, b, false); },
-        [](int, int, const uint4 (&)[Engine::NK]) {}, L.eng[wave]);
+        a, eng, npw, ctx, first, lookup, [](int, int, const uint4 (&)[Engine::NK]) {},
+        L.eng[wave]);
     eng.finish(L.eng[wave], L.m[wave], L.l[wave]);
     __syncthreads();
 

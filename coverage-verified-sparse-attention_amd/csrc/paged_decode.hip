@@ -40,7 +40,7 @@ __global__ void fill_zero_kernel(uint32_t *p, size_t n_words) {
 // at most kMaxSplits splits per head.  Verified and dense launches use the
 // stream-K grid of streamk_decode_kernel: target_workgroups(), fewer when
 // even the largest possible page list (every head walking all W pages) would
-// give a workgroup less than kMinPagesPerWg pages; the kernel narrows it to
+// give a workgroup less than kMinPagesPerSkWg pages; the kernel narrows it to
 // the pages actually walked.
 struct DecodeLaunch {
   bool streamk;
@@ -73,7 +73,7 @@ static DecodeLaunch plan_launch(int B, int H_kv, int max_sel, int W, bool listed
   }
   int64_t per_head = listed ? max_sel : 0;
   if (W > per_head) per_head = W;
-  int64_t g = (heads * per_head + kMinPagesPerWg - 1) / kMinPagesPerWg;
+  int64_t g = (heads * per_head + kMinPagesPerSkWg - 1) / kMinPagesPerSkWg;
   if (g > target) g = target;
   if (g < 1) g = 1;
   p.streamk = true;
