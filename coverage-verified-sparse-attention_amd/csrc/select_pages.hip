@@ -1588,10 +1588,9 @@ struct RunningLse {
 #pragma unroll
     for (int e = 0; e < N; ++e) s += fast_exp(v[e] - ref);
   }
-  // The sum relative to the block's maximum `to`.
-  __device__ __forceinline__ float rebased(float to) const {
-    return m == -INFINITY ? s : s * fast_exp(m - to);
-  }
+  // The sum relative to the block's maximum `to`: NaN where `to` is -inf (a
+  // full selection of pages without a score), as a sum of exp(v - to) is.
+  __device__ __forceinline__ float rebased(float to) const { return s * fast_exp(m - to); }
 };
 
 // check_coverage_kernel for rows wider than it holds in registers (W or

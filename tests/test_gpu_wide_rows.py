@@ -159,6 +159,27 @@ def test_check_coverage_wide(gpu, W, k):
         _gate_ok(acc.cpu(), cov.cpu(), wacc, wcov, tau)
 
 
+@pytest.mark.parametrize("W,k", [(4096, 64), (32769, 64), (70000, 8192)])
+def test_check_coverage_without_scores(gpu, W, k):
+    """Selected pages without a score: a selection that fills its power-of-two
+    block has no coverage (NaN, rejected at every tau), a shorter one none of
+    the row's; a row without any score likewise.  W <= 32768 is the register
+    kernel's answer to the same rows."""
+    ps = torch.randn(1, 4, W, generator=torch.Generator().manual_seed(W))
+    ps[0, :2, :k] = float("-inf")
+    ps[0, 2] = float("-inf")
+    ps[0, 3, :k:2] = float("-inf")
+    sel = torch.arange(k, dtype=torch.int32).expand(1, 4, k).contiguous()
+    nph = torch.tensor([[k, k - 1, k, k]], dtype=torch.int32)
+    wacc, wcov = ref.check_coverage(ps, sel, nph, 0.0)
+    assert wcov[0, 0].isnan() and not wacc[0, 0] and not wcov[0, 1].isnan()
+    acc, cov = ops.check_coverage(ps.to(gpu), sel.to(gpu), nph.to(gpu), 0.0)
+    assert torch.equal(cov.cpu().isnan(), wcov.isnan())
+    assert torch.equal(acc.cpu(), wacc)
+    some = ~wcov.isnan()
+    assert (cov.cpu()[some] - wcov[some]).abs().max().item() < COV_ATOL
+
+
 def test_select_budgeted_table_wide(gpu):
     """Per-row budgets (the static-table / adaptive path) ranked by separate
     scores, gated on the page scores, at W = 65536 and a narrower width."""
