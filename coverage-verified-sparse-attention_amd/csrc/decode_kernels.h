@@ -513,10 +513,11 @@ __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBu
 
 // ---------------------------------------------------------------- engines
 // A page engine owns one wave's softmax state for the G query heads of a KV
-// head and applies tiles to it.  One tile's K rows (kr) and V rows (vr) are
-// in registers at a time: each is staged to LDS as soon as it arrives and the
-// next tile's loads are issued into the same registers at once, so a wave
-// always has about one tile in flight; finish() leaves the wave's (o, m, l)
+// head and applies tiles to it.  The K rows (kr) and V rows (vr) of PD
+// tiles (one from D = 128 on) are in registers at a time: each tile is staged
+// to LDS as soon as it arrives and the loads of the tile PD further on are
+// issued into the same registers at once, so a wave always has about PD tiles
+// in flight; finish() leaves the wave's (o, m, l)
 // in LDS.
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -579,6 +580,11 @@ struct MfmaEngine {
   static constexpr int RPL = kWave / LPR;   // rows per wave load
   static constexpr int NL = kPageTokens / RPL;  // K (or V) loads per tile
   static constexpr int kRow = D + 8;        // LDS row of a K or V tile, in bf16
+  // Tiles in flight: 8 KiB of K and V or more.  Against the older engine (two
+  // tiles in flight at every D below 256, K in the operand layout) at D = 64:
+  // listed B = 1, 128K 15.3 -> 13.2 us, dense B = 4, 64K 99.2 -> 91.2, check
+  // B = 4, 64K 157.5 -> 147.9.
+  static constexpr int PD = D < 128 ? 128 / D : 1;
   struct Tiles {
     uint16_t k[kPageTokens * kRow], v[kPageTokens * kRow];
   };
@@ -594,7 +600,7 @@ struct MfmaEngine {
 
   float4_t o[NB];
   bf16x8_t qb[NK];
-  uint4 kr[NL], vr[NL];  // the tile in flight
+  uint4 kr[PD][NL], vr[PD][NL];  // the tiles in flight
   float m_g, l_g;
   int lane;
   int rmask;  // rows of a tile - 1: a load of row r reads row r & rmask
@@ -639,13 +645,14 @@ struct MfmaEngine {
     }
   }
 
-  // kr to the K tile, then back in the A operand layout (kop).  The row of a
+  // A tile's K rows to the K tile, then back in the A operand layout (kop).  The row of a
   // token appended by this launch (newrow, -1: none) comes from k_new.
   template <bool APP>
-  __device__ __forceinline__ void stage_k(Lds &lds, int newrow, const uint16_t *k_new) const {
+  __device__ __forceinline__ void stage_k(Lds &lds, const uint4 (&r)[NL], int newrow,
+                                          const uint16_t *k_new) const {
     uint16_t *dst = &lds.t.k[(lane / LPR) * kRow + 8 * (lane % LPR)];
 #pragma unroll
-    for (int i = 0; i < NL; ++i) *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = kr[i];
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = r[i];
     if (APP && newrow >= 0 && lane < LPR)
       *reinterpret_cast<uint4 *>(&lds.t.k[newrow * kRow + 8 * lane]) =
           *reinterpret_cast<const uint4 *>(k_new + 8 * lane);
@@ -656,19 +663,19 @@ struct MfmaEngine {
     for (int kk = 0; kk < NK; ++kk)
       kop[kk] = *reinterpret_cast<const uint4 *>(&lds.t.k[c16 * kRow + 32 * kk + 8 * grp]);
   }
-  // vr to the V tile (rows past the context are stored as zeros: the
+  // A tile's V rows to the V tile (rows past the context are stored as zeros: the
   // reference never reads them).
   template <bool APP>
-  __device__ __forceinline__ void stage_v(Lds &lds, int ntok, int newrow,
-                                          const uint16_t *v_new) {
+  __device__ __forceinline__ void stage_v(Lds &lds, uint4 (&r)[NL], int ntok, int newrow,
+                                          const uint16_t *v_new) const {
     uint16_t *dst = &lds.t.v[(lane / LPR) * kRow + 8 * (lane % LPR)];
     if (ntok < kPageTokens) {  // uniform: a sequence's last tile, or none
 #pragma unroll
       for (int i = 0; i < NL; ++i)
-        if (RPL * i + lane / LPR >= ntok) vr[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (RPL * i + lane / LPR >= ntok) r[i] = make_uint4(0u, 0u, 0u, 0u);
     }
 #pragma unroll
-    for (int i = 0; i < NL; ++i) *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = vr[i];
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = r[i];
     if (APP && newrow >= 0 && lane < LPR)
       *reinterpret_cast<uint4 *>(&lds.t.v[newrow * kRow + 8 * lane]) =
           *reinterpret_cast<const uint4 *>(v_new + 8 * lane);
@@ -802,7 +809,7 @@ struct TileChunk {
 };
 
 // One wave's walk over npw tiles.  `cur` is the first chunk's tiles, whose
-// first tile's loads are in flight (start_walk); chunk c's tiles come from
+// first PD tiles' loads are in flight (start_walk); chunk c's tiles come from
 // lookup(c) while chunk c - 1 is walked, so the loads run on across chunks.
 // score(lt, ntok, kop) sees each tile's keys first (SCORE).  APP: row new_off
 // of logical tile new_tile is the appended token's (k_new / v_new).
@@ -817,16 +824,19 @@ __device__ __forceinline__ void fetch_tile(const DecodeArgs &a, const Engine &en
 template <class Engine, bool APP = false>
 __device__ __forceinline__ void start_walk(const DecodeArgs &a, Engine &eng, const TileChunk &cur,
                                            int new_tile = -1, int new_off = -1) {
-  const int phys = __builtin_amdgcn_readlane(cur.phys, 0);
-  const int lt = __builtin_amdgcn_readlane(cur.lt, 0);
-  const int newrow = APP && lt == new_tile ? new_off : -1;
-  // K before V, here and in the walk: the wait for a tile's K then leaves its
-  // V in flight.
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.k_cache, eng.kr);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.v_cache, eng.vr);
-  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < Engine::PD; ++u) {
+    const int phys = __builtin_amdgcn_readlane(cur.phys, u);
+    const int lt = __builtin_amdgcn_readlane(cur.lt, u);
+    const int newrow = APP && lt == new_tile ? new_off : -1;
+    // K before V, here and in the walk: the wait for a tile's K then leaves
+    // its V in flight.
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.k_cache, eng.kr[u]);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.v_cache, eng.vr[u]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 template <class Engine, bool APP, bool SCORE, class Lookup, class Score>
@@ -836,32 +846,40 @@ __device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int
                                            int new_off = -1, const uint16_t *k_new = nullptr,
                                            const uint16_t *v_new = nullptr) {
   const int tl = Engine::tlog(a);
+  constexpr int PD = Engine::PD;
+  static_assert(kWave % PD == 0, "a chunk's tiles fill the slots evenly");
   TileChunk nxt;
-  int lt = __builtin_amdgcn_readlane(cur.lt, 0);
-  for (int e = 0; e < npw; ++e) {
+  int lt[PD];
+#pragma unroll
+  for (int u = 0; u < PD; ++u) lt[u] = __builtin_amdgcn_readlane(cur.lt, u);
+  for (int e = 0; e < npw; e += PD) {
     const int j = e & (kWave - 1);
     if (j == 0 && e + kWave < npw) nxt = lookup(e + kWave);
-    if (j == kWave - 1) {  // the next tile is the next chunk's first
+    if (j == kWave - PD) {  // the next tiles are the next chunk's first
       cur = nxt;
       nxt = TileChunk();
     }
-    // Lanes past the walk's end hold no tile.
-    const int phys_n = __builtin_amdgcn_readlane(cur.phys, (j + 1) & (kWave - 1));
-    const int lt_n = __builtin_amdgcn_readlane(cur.lt, (j + 1) & (kWave - 1));
-    const int newrow = APP && lt == new_tile ? new_off : -1;
-    const int newrow_n = APP && lt_n == new_tile ? new_off : -1;
-    const int ntok = min(1 << tl, max(0, ctx - (lt << tl)));
-    eng.template stage_k<APP>(lds, newrow, k_new);
-    fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.k_cache, eng.kr);
-    uint4 kop[Engine::NK];
-    eng.k_operand(lds, kop);
-    if constexpr (SCORE) score(lt, ntok, kop);
-    const bf16x8_t p = eng.softmax(kop, ntok, lds);
-    eng.template stage_v<APP>(lds, ntok, newrow, v_new);
-    fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr);
-    __builtin_amdgcn_sched_barrier(0);
-    eng.accumulate(p, lds);
-    lt = lt_n;
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {
+      if (PD > 1 && e + u >= npw) break;  // uniform
+      // Lanes past the walk's end hold no tile.
+      const int phys_n = __builtin_amdgcn_readlane(cur.phys, (j + u + PD) & (kWave - 1));
+      const int lt_n = __builtin_amdgcn_readlane(cur.lt, (j + u + PD) & (kWave - 1));
+      const int newrow = APP && lt[u] == new_tile ? new_off : -1;
+      const int newrow_n = APP && lt_n == new_tile ? new_off : -1;
+      const int ntok = min(1 << tl, max(0, ctx - (lt[u] << tl)));
+      eng.template stage_k<APP>(lds, eng.kr[u], newrow, k_new);
+      fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.k_cache, eng.kr[u]);
+      uint4 kop[Engine::NK];
+      eng.k_operand(lds, kop);
+      if constexpr (SCORE) score(lt[u], ntok, kop);
+      const bf16x8_t p = eng.softmax(kop, ntok, lds);
+      eng.template stage_v<APP>(lds, eng.vr[u], ntok, newrow, v_new);
+      fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr[u]);
+      __builtin_amdgcn_sched_barrier(0);
+      eng.accumulate(p, lds);
+      lt[u] = lt_n;
+    }
   }
 }
 
