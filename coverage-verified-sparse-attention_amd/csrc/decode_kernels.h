@@ -530,9 +530,12 @@ __device__ __forceinline__ uint32_t cvt_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
 }
 
-// No tile: ctx - (kNoTile << 4) < 0, so it has no valid token, and its loads
-// are dropped.
-constexpr int kNoTile = 1 << 26;
+// Logical tiles lie below kUnreadable.  kUnreadable + lt stands for tile lt of
+// a block outside the pool, kNoTile for no tile at all: neither has a valid
+// token (ctx - (kUnreadable << 4) < 0) and the loads of both are dropped.
+constexpr int kUnreadable = 1 << 26;
+constexpr int kNoTile = kUnreadable + (kUnreadable >> 1);
+static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 8 tiles at most");
 
 // MFMA engine: the G query heads (padded to 16) of a KV head against a tile
 // of 16 tokens are two small dense products for the matrix cores.
@@ -803,7 +806,7 @@ struct MfmaEngine {
 };
 
 // Tiles of a chunk of up to 64 of a wave's walk: lane j holds tile j's
-// physical tile and logical tile (kNoTile: none, nothing is read).
+// physical tile and logical tile (from kUnreadable on: nothing is read).
 struct TileChunk {
   int phys = 0, lt = kNoTile;
 };
@@ -818,7 +821,7 @@ __device__ __forceinline__ void fetch_tile(const DecodeArgs &a, const Engine &en
                                            int lt, int newrow, const uint16_t *cache,
                                            uint4 (&r)[Engine::NL]) {
   const int64_t base = (int64_t)phys * (eng.tile_bytes / 2);
-  eng.template fetch<APP>(cache + base, lt != kNoTile, newrow, r);
+  eng.template fetch<APP>(cache + base, lt < kUnreadable, newrow, r);
 }
 
 template <class Engine, bool APP = false>
@@ -1140,14 +1143,14 @@ __device__ __forceinline__ void listed_walk(const DecodeArgs &a, int split, int 
   }
   const int npw = max(0, (r1 - r0 - wave + NW - 1) / NW);
   // Tile `lane` of the chunk that starts at the wave's tile c0: its entry's
-  // logical tile and that tile's physical one, if both are valid.
+  // logical tile, if valid, and that tile's physical one.
   auto chunk = [&](int c0, int lt, int phys) {
     TileChunk c;
     if (APP && lt == nt.page && nt.new_blk >= 0) phys = nt.new_blk;
-    if (c0 + lane < npw && lt >= 0 && lt < (a.W << ts) && phys >= 0 &&
-        phys < (a.num_blocks << ts)) {
-      c.phys = phys;
-      c.lt = lt;
+    if (c0 + lane < npw && lt >= 0 && lt < (a.W << ts)) {
+      const bool readable = phys >= 0 && phys < (a.num_blocks << ts);
+      c.phys = readable ? phys : 0;
+      c.lt = readable ? lt : kUnreadable + lt;
     }
     return c;
   };
@@ -1167,7 +1170,10 @@ __device__ __forceinline__ void listed_walk(const DecodeArgs &a, int split, int 
         if constexpr (SCORE) {
           if (scoring) {
             const float sc = eng.page_score(kop, ntok, qrep);
-            if (lane == 0 && lt != kNoTile) a.spec_scores[(int64_t)bh * a.W + lt] = sc;
+            // A page whose block is outside the pool scores -inf, as the page
+            // scoring has it; the scoring workgroups leave it to this walk.
+            if (lane == 0 && lt != kNoTile)
+              a.spec_scores[(int64_t)bh * a.W + (lt & (kUnreadable - 1))] = sc;
           }
         }
       },

@@ -584,3 +584,49 @@ def test_selection_map_and_scores_over_a_schedule(gpu, shape):
         torch.cuda.synchronize()
         assert torch.equal(p.sel_map.cpu(), _map_of(p.page_indices, p.n_per_head, W, stride)), \
             (step, predict, tau)
+
+
+@pytest.mark.parametrize("tau", [0.0, 1.5])
+@pytest.mark.parametrize("predict", [1, 2, 0])
+@pytest.mark.parametrize("shape", [(8, 4), (16, 2)])
+def test_check_scores_blocks_outside_the_pool(gpu, shape, predict, tau):
+    """Table entries outside the pool appear between two checks of a plan
+    (a sequence rolled back under its cached selection): the second check
+    scores their pages -inf, whoever scores them, and equals the separate
+    kernels bit for bit.  Among the bad pages: the first and the last, one of
+    every row's selection and one outside the first row's."""
+    H, G = shape
+    inp, W, budget = _inputs(gpu, h=H, g=G)
+    ctx, bt = inp.context_lens, inp.block_tables.clone()
+    ps0 = ops.score_pages(inp.q, inp.k_cache, bt, ctx, H, G, 16)
+    sel0, nph0 = ops.select_topk(ps0, budget, ctx, 16)
+    stats = torch.zeros(6, dtype=torch.int64, device=gpu)
+    work = torch.zeros(2, dtype=torch.int64, device=gpu)
+    plan = ops.StepPlan(inp.q, inp.k_cache, inp.v_cache, bt, ctx, H, G, 16, budget, tau,
+                        sel0.clone(), nph0.clone(), ps0.clone(), stats, work)
+    plan.run(_lib.STEP_LAZY_CHECK, inp.q)  # page_scores: finite on every valid page
+    pages = (ctx + 15) // 16
+    for b in range(2):
+        n = int(pages[b])
+        picked = plan.page_indices[b, 0].tolist()
+        bad = {0, n - 1, next(p for p in range(n // 2, n) if p not in picked)}
+        bad |= {int(plan.page_indices[b, h, h]) for h in range(H)}
+        for i, p in enumerate(sorted(bad)):
+            bt[b, p] = (-1, inp.k_cache.shape[0], -(1 << 30), 1 << 30)[i % 4]
+    q1 = jitter_query(inp.q, 0.5, 4)
+    sel, nph = plan.page_indices.clone(), plan.n_per_head.clone()
+    cache, stats_r, work_r = ps0.clone(), stats.clone(), work.clone()
+    plan.spec_state[0] = predict
+    got = plan.run(_lib.STEP_LAZY_CHECK, q1)
+    assert int(plan.spec_state[1]) == predict
+    ps = ops.score_pages(q1, inp.k_cache, bt, ctx, H, G, 16)
+    chk, cov = ops.check_coverage(ps, sel, nph, tau)
+    acc = ops.select_or_keep(ps, chk, budget, ctx, 16, tau, sel, nph, cov, cache, stats_r)
+    want = ops.verified_decode(q1, inp.k_cache, inp.v_cache, bt, ctx, sel, nph, acc, H, G, 16,
+                               output_dtype=q1.dtype, work=work_r)
+    assert bool(torch.isinf(ps[0, :, 0]).all()) and bool(acc.all()) == (tau == 0.0)
+    assert torch.equal(plan.page_scores, ps)
+    assert torch.equal(plan.accept.view(torch.bool), acc)
+    assert torch.equal(plan.page_indices, sel) and torch.equal(plan.n_per_head, nph)
+    assert torch.equal(got, want)
+    assert torch.equal(stats, stats_r) and torch.equal(work, work_r)
