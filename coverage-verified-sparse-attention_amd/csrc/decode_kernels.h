@@ -1204,9 +1204,13 @@ __global__ __launch_bounds__(NW * kWave, walk_waves(Engine::kD)) void listed_dec
 // sequence's first head also moves its context length, page-table entry
 // and allocation count as cvsa_append_kv does.  Later launches see the
 // appended cache.
+// Three waves per SIMD (142 registers): at walk_waves' four (128) every
+// instance spilled 1 or 2 of them to scratch, and no launch was faster for the
+// fourth wave (8185 tokens, budget 25%, cold caches: B = 1 12.1 -> 11.8 us,
+// B = 32 48.5 -> 47.6, B = 128 176.6 -> 173.9).
 template <int G, class Engine, int NW>
-__global__ __launch_bounds__(NW * kWave, walk_waves(Engine::kD)) void listed_append_kernel(const DecodeArgs a,
-                                                                   const AppendArgs app) {
+__global__ __launch_bounds__(NW * kWave, 3) void listed_append_kernel(const DecodeArgs a,
+                                                                      const AppendArgs app) {
   static_assert(Engine::kD == 128, "the fused append is built for D = 128");
   __shared__ WalkLds<G, Engine, NW> L;
   const int lane = threadIdx.x & 63;
