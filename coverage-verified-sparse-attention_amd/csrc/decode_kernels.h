@@ -273,10 +273,10 @@ __device__ __forceinline__ int approx_booked_pages(const DecodeArgs &a, int bh, 
 }
 
 // Stream-K partition.  The heads' page walks are concatenated (head-major)
-// into one list of T pages and cut into n_wg equal ranges; workgroup w owns
-// pages [start(w), start(w + 1)), start(w) = floor(w * T / n_wg).  n_wg is the
-// launch size, reduced so that a workgroup gets at least kMinPagesPerSkWg
-// pages.  T < 2^31 and n_wg <= kMaxSplits, so every quantity is computed in
+// into one list of T tiles and cut into n_wg equal ranges; workgroup w owns
+// tiles [start(w), start(w + 1)), start(w) = floor(w * T / n_wg).  n_wg is the
+// launch size, reduced so that a workgroup gets at least kMinTilesPerSkWg
+// tiles.  T < 2^31 and n_wg <= kMaxSplits, so every quantity is computed in
 // 32 bits (64-bit division is a long instruction sequence on the GPU).
 constexpr int kMaxHeads = 4096;  // B * H_kv of one launch
 // Two-level merge of a stream-K head with more than kTwoLevelMin partials:
@@ -291,16 +291,18 @@ constexpr int kMergeGroup = 16;
 constexpr int kTwoLevelMin = 48;
 constexpr int kGroupCounters = 2 * 256;  // 2 x the largest stream-K grid
 constexpr int kMinPagesPerWg = kMinPagesPerWave * kWavesPerWg;
-// A stream-K workgroup takes at least this many pages, so a short launch has
-// fewer partials to hand off (a scoring step at B = 1, 8K, five of eight heads
-// recovered, 2944 pages: 8 pages per workgroup 29.2 us, 16 26.4, 24 30.4,
-// 32 28.0).
-constexpr int kMinPagesPerSkWg = 2 * kMinPagesPerWg;
+// A stream-K workgroup takes at least this many tiles, so a short launch has
+// fewer partials to hand off.  us a step with 8 / 16 / 32 (16-token pages,
+// H_kv = 8, G = 4): scoring steps that recover half the heads, B = 1, 1K tokens
+// 20.1 / 21.9 / 28.0, 4K 22.9 / 23.1 / 26.5, 8K 29.1 / 26.4 / 28.0, 16K 34.8 /
+// 34.8 / 33.9, B = 4, 2K 26.5 / 24.4 / 27.7; dense 1K to 4K 12.0-12.4 /
+// 12.0-12.3 / 14.4-14.7, from 8K on the same.
+constexpr int kMinTilesPerSkWg = 2 * kMinPagesPerWg;
 
 struct Partition {
-  int T, n, q, r;  // pages, workgroups, T / n, T % n
+  int T, n, q, r;  // tiles, workgroups, T / n, T % n
   __device__ __forceinline__ Partition(int T_, int grid) : T(T_) {
-    n = max(1, min(grid, (T + kMinPagesPerSkWg - 1) / kMinPagesPerSkWg));
+    n = max(1, min(grid, (T + kMinTilesPerSkWg - 1) / kMinTilesPerSkWg));
     q = T / n;
     r = T - q * n;
   }

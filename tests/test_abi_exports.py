@@ -81,6 +81,26 @@ def test_decode_workspace_layout_is_fixed():
     assert lib.cvsa_decode_workspace_bytes(1, 32, 8, 96, 64, 8192, 1) == 0
 
 
+def test_dense_grid_per_block_size():
+    """Workgroups of a dense launch by block size (read from the workspace a
+    call without one asks for: a partial row per workgroup and head): one per
+    16 pages of one tile (8 and 16 tokens), one per 8 pages of several tiles,
+    256 at most; cvsa_decode_workspace_bytes covers every block size."""
+    lib = _lib_or_skip()
+    H_kv, G, D, tokens = 8, 4, 128, 8192
+    p = range(1 << 20, 1 << 30, 1 << 16)
+    for bs in (8, 16, 32, 64, 128):
+        W = tokens // bs
+        rc = lib.cvsa_dense_decode(p[0], H_kv * G * D, D, p[1], p[2], 2 * W, p[3], W, p[4], 1,
+                                   H_kv * G, H_kv, D, bs, W, None, None, None, p[5],
+                                   _lib.DTYPE_BF16, None, None, 0, None)
+        assert rc == _lib.CVSA_ERR_WORKSPACE
+        need = int(re.search(rb"workspace of (\d+) bytes", lib.cvsa_last_error())[1])
+        rows = (need - 18432) // (G * (D + 4) * 4)
+        assert rows - H_kv == min(256, H_kv * W // (16 if bs <= 16 else 8)), bs
+        assert need <= lib.cvsa_decode_workspace_bytes(1, H_kv * G, H_kv, D, 0, W, 1), bs
+
+
 def _step_desc(**over):
     """A well-formed step descriptor over fake (never dereferenced) pointers."""
     fake = iter(range(1 << 20, 1 << 30, 1 << 16))
