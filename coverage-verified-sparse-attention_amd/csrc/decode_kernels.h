@@ -275,8 +275,8 @@ __device__ __forceinline__ int approx_booked_pages(const DecodeArgs &a, int bh, 
 // Stream-K partition.  The heads' page walks are concatenated (head-major)
 // into one list of T tiles and cut into n_wg equal ranges; workgroup w owns
 // tiles [start(w), start(w + 1)), start(w) = floor(w * T / n_wg).  n_wg is the
-// launch size, reduced so that a workgroup gets at least kMinTilesPerSkWg
-// tiles.  T < 2^31 and n_wg <= kMaxSplits, so every quantity is computed in
+// launch size, reduced so that a workgroup gets at least min_sk_tiles tiles.
+// T < 2^31 and n_wg <= kMaxSplits, so every quantity is computed in
 // 32 bits (64-bit division is a long instruction sequence on the GPU).
 constexpr int kMaxHeads = 4096;  // B * H_kv of one launch
 // Two-level merge of a stream-K head with more than kTwoLevelMin partials:
@@ -296,13 +296,17 @@ constexpr int kMinPagesPerWg = kMinPagesPerWave * kWavesPerWg;
 // H_kv = 8, G = 4): scoring steps that recover half the heads, B = 1, 1K tokens
 // 20.1 / 21.9 / 28.0, 4K 22.9 / 23.1 / 26.5, 8K 29.1 / 26.4 / 28.0, 16K 34.8 /
 // 34.8 / 33.9, B = 4, 2K 26.5 / 24.4 / 27.7; dense 1K to 4K 12.0-12.4 /
-// 12.0-12.3 / 14.4-14.7, from 8K on the same.
+// 12.0-12.3 / 14.4-14.7, from 8K on the same.  Approximate recovery walks
+// lists of a like length per head and takes 8 (budget 5%, expanded 30%: 1K
+// 24.3 / 25.7 / 31.6, 4K 24.4 / 26.4 / 32.7, 16K 31.8 / 33.8 / 36.3; 64-token
+// pages 4K 26.4 / 30.9 / 34.6).
 constexpr int kMinTilesPerSkWg = 2 * kMinPagesPerWg;
+constexpr int min_sk_tiles(bool approx) { return approx ? kMinPagesPerWg : kMinTilesPerSkWg; }
 
 struct Partition {
   int T, n, q, r;  // tiles, workgroups, T / n, T % n
-  __device__ __forceinline__ Partition(int T_, int grid) : T(T_) {
-    n = max(1, min(grid, (T + kMinTilesPerSkWg - 1) / kMinTilesPerSkWg));
+  __device__ __forceinline__ Partition(int T_, int grid, int min_tiles) : T(T_) {
+    n = max(1, min(grid, (T + min_tiles - 1) / min_tiles));
     q = T / n;
     r = T - q * n;
   }
@@ -1473,7 +1477,7 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
   lds_barrier();  // s_start and s_listed
   T = __builtin_amdgcn_readfirstlane(T);
 
-  const Partition part(max(T, 1), a.sk_grid);
+  const Partition part(max(T, 1), a.sk_grid, min_sk_tiles(MODE == kModeApprox));
   const int n_wg = T > 0 ? part.n : a.sk_grid;
   if (w >= n_wg) return;  // uniform
 

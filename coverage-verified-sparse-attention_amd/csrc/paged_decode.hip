@@ -40,12 +40,12 @@ __global__ void fill_zero_kernel(uint32_t *p, size_t n_words) {
 // at most kMaxSplits splits per head.  Verified and dense launches use the
 // stream-K grid of streamk_decode_kernel: kTargetWorkgroups, fewer when
 // even the largest possible page list (every head walking all W pages) would
-// give a workgroup less than kMinTilesPerSkWg one-tile pages, or less than
+// give a workgroup less than min_sk_tiles one-tile pages, or less than
 // kMinPagesPerWg pages of several tiles (2^ts of them: 16 to 64 tiles); the
 // kernel narrows it to the tiles actually walked.  Pages of several tiles do
-// not get one workgroup per kMinTilesPerSkWg tiles: callers size the
+// not get one workgroup per min_sk_tiles tiles: callers size the
 // workspace without the block size, for a workgroup per kMinPagesPerWg pages.
-// (One per kMinTilesPerSkWg such pages took a dense 8K call, H_kv = 8, from
+// (One per 16 such pages took a dense 8K call, H_kv = 8, from
 // 16.3 to 23.1 us with 64-token pages and from 23.2 to 36.8 with 128-token
 // ones.)
 struct DecodeLaunch {
@@ -58,7 +58,7 @@ struct DecodeLaunch {
 };
 
 static DecodeLaunch plan_launch(int B, int H_kv, int max_sel, int W, bool listed,
-                                bool all_pages, int ts) {
+                                bool all_pages, int ts, bool approx) {
   const int64_t heads = (int64_t)B * H_kv;
   const int target = kTargetWorkgroups;
   DecodeLaunch p{};
@@ -79,7 +79,7 @@ static DecodeLaunch plan_launch(int B, int H_kv, int max_sel, int W, bool listed
   }
   int64_t per_head = listed ? max_sel : 0;
   if (W > per_head) per_head = W;
-  const int min_pages = ts == 0 ? kMinTilesPerSkWg : kMinPagesPerWg;
+  const int min_pages = ts == 0 ? min_sk_tiles(approx) : kMinPagesPerWg;
   int64_t g = (heads * per_head + min_pages - 1) / min_pages;
   if (g > target) g = target;
   if (g < 1) g = 1;
@@ -91,7 +91,7 @@ static DecodeLaunch plan_launch(int B, int H_kv, int max_sel, int W, bool listed
   if (listed) {
     // Verified launches also carry the listed partition, which they run
     // when every head is accepted: at least one workgroup per (split, head).
-    const DecodeLaunch lp = plan_launch(B, H_kv, max_sel, W, true, false, ts);
+    const DecodeLaunch lp = plan_launch(B, H_kv, max_sel, W, true, false, ts, approx);
     p.pps = lp.pps;
     p.n_splits = lp.n_splits;
     const int64_t n_listed = (int64_t)lp.grid_x * lp.grid_y;
@@ -99,7 +99,7 @@ static DecodeLaunch plan_launch(int B, int H_kv, int max_sel, int W, bool listed
     if (lp.partial_rows > p.partial_rows) p.partial_rows = lp.partial_rows;
     // ... and the identity partition, which they run when every head is
     // rejected: the listed partition of a W-page list.
-    const DecodeLaunch ip = plan_launch(B, H_kv, W, W, true, false, ts);
+    const DecodeLaunch ip = plan_launch(B, H_kv, W, W, true, false, ts, approx);
     p.pps_all = ip.pps;
     p.n_splits_all = ip.n_splits;
     const int64_t n_ident = (int64_t)ip.grid_x * ip.grid_y;
@@ -122,11 +122,11 @@ static_assert(kTargetWorkgroups * 2 <= kGroupCounters, "a group counter per grou
 static_assert(kCounterAreaBytes % 256 == 0, "partial rows start 256-byte aligned");
 
 static size_t workspace_bytes_for(int B, int H_q, int H_kv, int D, int max_sel, int W,
-                                  bool listed, bool all_pages, int ts) {
+                                  bool listed, bool all_pages, int ts, bool approx) {
   // One launch serves at most kMaxGroup query heads per KV head; larger
   // groups run as several launches over the same workspace.
   const int G = min(H_q / H_kv, kMaxGroup);
-  const DecodeLaunch p = plan_launch(B, H_kv, max_sel, W, listed, all_pages, ts);
+  const DecodeLaunch p = plan_launch(B, H_kv, max_sel, W, listed, all_pages, ts, approx);
   if (p.partial_rows == 0) return 0;
   return kCounterAreaBytes + p.partial_rows * G * part_stride(D) * sizeof(float);
 }
@@ -190,11 +190,13 @@ static int validate_decode(const char *name, DecodeArgs &a, int B, int H_q, int 
                                     a.out_dtype <= CVSA_DTYPE_FP32),
                CVSA_ERR_INVALID, "%s: bad output dtype %d", name, a.out_dtype);
 
-  p = plan_launch(B, H_kv, listed ? a.max_sel : 0, W, listed, all_pages, ts);
+  const bool approx = a.alt_idx != nullptr;
+  p = plan_launch(B, H_kv, listed ? a.max_sel : 0, W, listed, all_pages, ts, approx);
   CVSA_REQUIRE((!p.streamk && p.partial_rows == 0) || (int64_t)B * H_kv <= kMaxHeads,
                CVSA_ERR_UNSUPPORTED, "%s: B * H_kv = %lld exceeds %d heads per launch", name,
                (long long)B * H_kv, kMaxHeads);
-  need = workspace_bytes_for(B, H_q, H_kv, D, listed ? a.max_sel : 0, W, listed, all_pages, ts);
+  need = workspace_bytes_for(B, H_q, H_kv, D, listed ? a.max_sel : 0, W, listed, all_pages, ts,
+                             approx);
   CVSA_REQUIRE(need == 0 || need - kCounterAreaBytes < ((size_t)1 << 31),
                CVSA_ERR_UNSUPPORTED,
                "%s: %zu bytes of split partials exceed the 2 GiB buffer range", name,
@@ -317,7 +319,8 @@ extern "C" size_t cvsa_decode_workspace_bytes(int32_t B, int32_t H_q, int32_t H_
     return 0;
   const bool listed = max_sel_pages > 0;
   // Any block size: pages of several tiles take the most workgroups.
-  return workspace_bytes_for(B, H_q, H_kv, D, max_sel_pages, W, listed, all_pages != 0, 1);
+  return workspace_bytes_for(B, H_q, H_kv, D, max_sel_pages, W, listed, all_pages != 0, 1,
+                             false);
 }
 
 extern "C" int cvsa_workspace_init(void *workspace, size_t workspace_bytes, void *stream) {
@@ -612,10 +615,10 @@ int score_and_speculate(const uint16_t *q, int64_t q_stride_b, int64_t q_stride_
   // The speculative dense decode walks the identity partition (a listed
   // walk of a W-page list), as a verified launch whose heads are all
   // rejected does.
-  const DecodeLaunch ip = plan_launch(B, H_kv, W, W, true, false, a.ts);
+  const DecodeLaunch ip = plan_launch(B, H_kv, W, W, true, false, a.ts, false);
   a.pps_all = ip.pps << a.ts;
   a.n_splits_all = ip.n_splits;
-  const size_t need_ident = workspace_bytes_for(B, H_q, H_kv, D, W, W, true, false, a.ts);
+  const size_t need_ident = workspace_bytes_for(B, H_q, H_kv, D, W, W, true, false, a.ts, false);
   if (need_ident > need) need = need_ident;
   if ((rc = check_workspace(name, workspace, workspace_bytes, need)) != CVSA_OK) return rc;
   bind_workspace(a, workspace, need);
