@@ -73,9 +73,6 @@ constexpr int kMaxSplits = 256;            // partials per head (and workgroups 
 // dense at B = 4, 64K 186 against 178 us.
 constexpr int kWavesPerWg = 4;
 constexpr int kMinPagesPerWave = 2;        // pages per wave of a split, at least
-// Waves per SIMD the listed kernels' registers are held to: launches of more
-// than one workgroup per CU overlap one's hand-off with another's walk.
-constexpr int walk_waves(int D) { return D > 128 ? 2 : 4; }
 
 struct DecodeArgs {
   const uint16_t *q;
@@ -94,7 +91,7 @@ struct DecodeArgs {
   int H_kv, W;
   int D;      // head dimension (the launch's engine is compiled for it)
   int ts;     // tiles per page = 1 << ts
-  int tl;     // rows of a tile = 1 << tl: 4, or 3 for 8-token pages
+  int tl;     // rows of a tile = 1 << tl: 4, or 3 for 8-token pages (picks the engine)
   // Query heads: the launch serves heads q_off .. q_off + G - 1 (G the
   // kernel's group, at most 16) of each KV head's group of q_group; a larger
   // group runs as one launch per 16 of its heads.
@@ -572,28 +569,43 @@ static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 
 // engine of two tiles in flight the kernels took: listed 19.1 -> 17.1 us at
 // cfg3, 47.2 -> 43.2 us at B = 32 (ragged 8K), 10.3 -> 9.0 us at B = 1, 8K;
 // dense at B = 4, 64K, G = 8 185-191 -> 178 us.
-template <int G, int D, int TS>
+//
+// PAGES: kPages16 (one 16-row tile per page), kPagesWide (2^ts of them) or
+// kPages8.  An 8-token page is a tile of 8 rows: rows 8 .. 15 of the two LDS
+// tiles are no token's (K: never looked at, V: zeros), are not read from
+// memory, and twice as many tiles are in flight.  With 16-row loads folded
+// onto the 8 rows and one tile in flight at D = 128 -> as here, H_kv = 8, G = 4:
+// listed B = 1, 128K 25.0 -> 19.9 us, B = 32 (ragged 8K) 71.0 -> 49.5; dense
+// B = 4, 64K 261.2 -> 186.2.
+enum { kPages16, kPagesWide, kPages8 };
+template <int G, int D, int PAGES>
 struct MfmaEngine {
   static_assert(G <= 16, "GQA group larger than the MFMA tile");
   static_assert(D == 32 || D == 64 || D == 128 || D == 256, "head dimension");
-  static_assert(TS == 0 || TS == -1, "tile shift: 0 (16-token pages) or -1 (from the args)");
   static constexpr int kD = D;
-  static constexpr int kTileShift = TS;  // -1: from the args
-  // Tiles per page = 1 << tshift(a), rows per tile = 1 << tlog(a): compiled
-  // in for 16-token pages.
-  static __device__ __forceinline__ int tshift(const DecodeArgs &a) { return TS >= 0 ? TS : a.ts; }
-  static __device__ __forceinline__ int tlog(const DecodeArgs &a) { return TS >= 0 ? 4 : a.tl; }
+  static constexpr int kPages = PAGES;
+  // Tiles per page = 1 << tshift(a), rows per tile kRows = 1 << kRowsLog.
+  static __device__ __forceinline__ int tshift(const DecodeArgs &a) {
+    return PAGES == kPagesWide ? a.ts : 0;
+  }
+  static constexpr int kRowsLog = PAGES == kPages8 ? 3 : 4;
+  static constexpr int kRows = 1 << kRowsLog;
   static constexpr int NK = D / 32;         // S = K Q^T MFMAs (32 dimensions each)
   static constexpr int NB = D / 16;         // O column blocks (16 dimensions each)
   static constexpr int LPR = D / 8;         // lanes per K or V row (16 bytes each)
   static constexpr int RPL = kWave / LPR;   // rows per wave load
-  static constexpr int NL = kPageTokens / RPL;  // K (or V) loads per tile
+  static constexpr int NL = kRows > RPL ? kRows / RPL : 1;  // K (or V) loads per tile
   static constexpr int kRow = D + 8;        // LDS row of a K or V tile, in bf16
   // Tiles in flight: 8 KiB of K and V or more.  Against the older engine (two
   // tiles in flight at every D below 256, K in the operand layout) at D = 64:
   // listed B = 1, 128K 15.3 -> 13.2 us, dense B = 4, 64K 99.2 -> 91.2, check
   // B = 4, 64K 157.5 -> 147.9.
-  static constexpr int PD = D < 128 ? 128 / D : 1;
+  static constexpr int PD = kRows * D < 2048 ? 2048 / (kRows * D) : 1;
+  static_assert(PD * kRows * D * 4 >= 8192, "8 KiB of K and V in flight per wave");
+  // Waves per SIMD the listed decode's registers are held to: launches of more
+  // than one workgroup per CU overlap one's hand-off with another's walk.
+  // (8-token pages at D = 128 spill 27 registers at four.)
+  static constexpr int kWalkWaves = D > 128 ? 2 : D == 128 && PAGES == kPages8 ? 3 : 4;
   struct Tiles {
     uint16_t k[kPageTokens * kRow], v[kPageTokens * kRow];
   };
@@ -612,18 +624,17 @@ struct MfmaEngine {
   uint4 kr[PD][NL], vr[PD][NL];  // the tiles in flight
   float m_g, l_g;
   int lane;
-  int rmask;  // rows of a tile - 1: a load of row r reads row r & rmask
   uint32_t voff, row_bytes, tile_bytes;
   float scale;
 
   __device__ __forceinline__ void init(const DecodeArgs &a, int b, int h, int lane_) {
     lane = lane_;
     scale = a.scale;
-    rmask = (1 << tlog(a)) - 1;
     row_bytes = (uint32_t)(a.H_kv * D * 2);
-    tile_bytes = row_bytes << tlog(a);
+    tile_bytes = row_bytes << kRowsLog;
     const int c16 = lane & 15, grp = lane >> 4;
-    voff = ((lane / LPR) & rmask) * row_bytes + (uint32_t)(h * D + 8 * (lane % LPR)) * 2;
+    voff = (lane / LPR) * row_bytes + (uint32_t)(h * D + 8 * (lane % LPR)) * 2;
+    if (RPL > kRows && lane / LPR >= kRows) voff = kRegionSkip;  // no row of the tile
     // Rows past the group repeat head G-1: MFMA output rows are independent
     // and those rows are never written out.  No select on the loaded value,
     // so nothing waits for q before the first tile is consumed.
@@ -639,9 +650,8 @@ struct MfmaEngine {
   }
 
   // The rows of the tile at `base` (wave-uniform) into r.  No tile (live
-  // false): nothing is read.  Load i reads rows RPL i + lane / LPR: with
-  // 8-row tiles those past row 7 fold onto rows 0..7 (RPL is a power of two,
-  // so the mask splits).  The lanes of row `newrow` (-1: none) read nothing.
+  // false): nothing is read.  Load i reads rows RPL i + lane / LPR.  The
+  // lanes of row `newrow` (-1: none) read nothing.
   template <bool APP>
   __device__ __forceinline__ void fetch(const uint16_t *base, bool live, int newrow,
                                         uint4 (&r)[NL]) const {
@@ -650,8 +660,17 @@ struct MfmaEngine {
     for (int i = 0; i < NL; ++i) {
       uint32_t oi = off;
       if (APP && RPL * i + lane / LPR == newrow) oi = kRegionSkip;
-      r[i] = region_load16(base, tile_bytes, oi, ((RPL * i) & rmask) * row_bytes);
+      r[i] = region_load16(base, tile_bytes, oi, RPL * i * row_bytes);
     }
+  }
+
+  // Zeros for the V rows that no load of an 8-row tile covers, before a walk:
+  // their weights are zero, and the rows stay as they are until finish().
+  __device__ __forceinline__ void clear_v_tail(Lds &lds) const {
+    uint16_t *dst = &lds.t.v[(lane / LPR) * kRow + 8 * (lane % LPR)];
+#pragma unroll
+    for (int i = NL; i < kPageTokens / RPL; ++i)
+      *reinterpret_cast<uint4 *>(dst + RPL * i * kRow) = make_uint4(0u, 0u, 0u, 0u);
   }
 
   // A tile's K rows to the K tile, then back in the A operand layout (kop).  The row of a
@@ -678,7 +697,7 @@ struct MfmaEngine {
   __device__ __forceinline__ void stage_v(Lds &lds, uint4 (&r)[NL], int ntok, int newrow,
                                           const uint16_t *v_new) const {
     uint16_t *dst = &lds.t.v[(lane / LPR) * kRow + 8 * (lane % LPR)];
-    if (ntok < kPageTokens) {  // uniform: a sequence's last tile, or none
+    if (ntok < kRows) {  // uniform: a sequence's last tile, or none
 #pragma unroll
       for (int i = 0; i < NL; ++i)
         if (RPL * i + lane / LPR >= ntok) r[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -854,9 +873,10 @@ __device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int
                                            typename Engine::Lds &lds, int new_tile = -1,
                                            int new_off = -1, const uint16_t *k_new = nullptr,
                                            const uint16_t *v_new = nullptr) {
-  const int tl = Engine::tlog(a);
+  constexpr int tl = Engine::kRowsLog;
   constexpr int PD = Engine::PD;
   static_assert(kWave % PD == 0, "a chunk's tiles fill the slots evenly");
+  eng.clear_v_tail(lds);
   TileChunk nxt;
   int lt[PD];
 #pragma unroll
@@ -1120,7 +1140,7 @@ __device__ __forceinline__ void listed_walk(const DecodeArgs &a, int split, int 
   const int n_spl = IDENT ? a.n_splits_all : a.n_splits;
   const int32_t *idx_row = a.page_idx + (int64_t)bh * a.idx_stride;
   const int ts = Engine::tshift(a);
-  const int tl = Engine::tlog(a);
+  constexpr int tl = Engine::kRowsLog;
   // IDENT: entry e is tile e of the head's valid pages (n_valid as the
   // reference computes it, at most W).
   const int n = IDENT ? max(0, min(valid_pages_sh(ctx, tl + ts), a.W)) << ts
@@ -1193,7 +1213,8 @@ __device__ __forceinline__ void listed_walk(const DecodeArgs &a, int split, int 
 
 // The listed decode: a static grid of (split, head) workgroups.
 template <int G, class Engine, int NW>
-__global__ __launch_bounds__(NW * kWave, walk_waves(Engine::kD)) void listed_decode_kernel(const DecodeArgs a) {
+__global__ __launch_bounds__(NW * kWave, Engine::kWalkWaves) void listed_decode_kernel(
+    const DecodeArgs a) {
   __shared__ WalkLds<G, Engine, NW> L;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1210,7 +1231,7 @@ __global__ __launch_bounds__(NW * kWave, walk_waves(Engine::kD)) void listed_dec
 // sequence's first head also moves its context length, page-table entry
 // and allocation count as cvsa_append_kv does.  Later launches see the
 // appended cache.
-// Three waves per SIMD (142 registers): at walk_waves' four (128) every
+// Three waves per SIMD (142 registers): at the listed decode's four (128) every
 // instance spilled 1 or 2 of them to scratch, and no launch was faster for the
 // fourth wave (8185 tokens, budget 25%, cold caches: B = 1 12.1 -> 11.8 us,
 // B = 32 48.5 -> 47.6, B = 128 176.6 -> 173.9).
@@ -1294,7 +1315,7 @@ constexpr int kSpecHeadPPW = 16;
 // at once.  Reading the kept selection's keys once: kept check 64.0 -> 61.1 us
 // at cfg3 (16 pages per scoring wave; 8 and 32 measured 61.2 and 62.0).
 template <int G, class Engine, int NW>
-__global__ __launch_bounds__(NW * kWave, Engine::kTileShift != 0 ? 2 : G > 8 ? 3 : 4)
+__global__ __launch_bounds__(NW * kWave, Engine::kPages != kPages16 ? 2 : G > 8 ? 3 : 4)
 void score_spec_kernel(const DecodeArgs a, const ScoreArgs s, int score_gx) {
   __shared__ WalkLds<G, Engine, NW> L;
   __shared__ uint4 s_qrep[NW][16];  // decode part: q_rep per wave
@@ -1307,12 +1328,12 @@ void score_spec_kernel(const DecodeArgs a, const ScoreArgs s, int score_gx) {
   // keys (16-token pages and a selection map), else 0.
   const int pred = __builtin_amdgcn_readfirstlane(a.spec_state[0]);
   const int go = pred == 1 ? 1
-                 : pred == 2 && Engine::kTileShift == 0 && a.spec_scores != nullptr ? 2
+                 : pred == 2 && Engine::kPages == kPages16 && a.spec_scores != nullptr ? 2
                                                                                     : 0;
   if (w >= n_dec) {  // uniform
     const int sw = w - n_dec;
     const int gw = (sw % score_gx) * NW + wave, b = sw / score_gx;
-    if constexpr (Engine::kTileShift == 0) {
+    if constexpr (Engine::kPages == kPages16) {
       // With a skip map, the pages the speculative decode walks (when it
       // runs) are scored there: the selection's, or every valid page.
       const int ctx = __builtin_amdgcn_readfirstlane(s.context_lens[b]);
@@ -1330,9 +1351,9 @@ void score_spec_kernel(const DecodeArgs a, const ScoreArgs s, int score_gx) {
     const int bh = w / a.n_splits;
     int lp, phys;
     listed_first_pages<NW>(a, split, bh, wave, lane, Engine::tshift(a), lp, phys);
-    listed_walk<G, Engine, NW, false, Engine::kTileShift == 0>(a, split, bh, lp, phys, L,
+    listed_walk<G, Engine, NW, false, Engine::kPages == kPages16>(a, split, bh, lp, phys, L,
                                                                    NewToken(), s_qrep[wave]);
-  } else if constexpr (Engine::kTileShift == 0) {
+  } else if constexpr (Engine::kPages == kPages16) {
     if (go != 2 || w >= a.n_splits_all * a.heads) return;  // uniform
     const int split = w % a.n_splits_all;
     const int bh = w / a.n_splits_all;
@@ -1371,7 +1392,7 @@ __global__ __launch_bounds__(NW * kWave, Engine::kD > 128 ? 1 : 2) void streamk_
   const int heads = a.heads;
   constexpr int D = Engine::kD;
   const int ts = Engine::tshift(a);
-  const int tl = Engine::tlog(a);
+  constexpr int tl = Engine::kRowsLog;
 
   // Tiles per head, scanned into their exclusive prefix in s_start, one head
   // per thread and pass of NT heads (loads issued without a branch, index
@@ -1564,14 +1585,14 @@ constexpr int kTargetWorkgroups = 256;
 static_assert(kTargetWorkgroups <= kMaxSplits, "one merge per head fits the merge LDS");
 
 // Launches of a validated decode for GQA group size G, explicitly
-// instantiated per G in the decode_g*.hip files (one translation unit per
-// four group sizes, so the library's objects compile in parallel). 
+// instantiated per G in the decode_g*.hip and decode_pages8_g*.hip files (one
+// translation unit per four group sizes, so the objects compile in parallel).
 enum { kLaunchListed = 0, kLaunchVerified = 1, kLaunchAll = 2, kLaunchApprox = 3 };
 
-template <int G, int D, int TS>
-void launch_decode_gdt(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
+template <int G, int D, int PAGES>
+void launch_decode_gdp(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
   const dim3 block(kWavesPerWg * kWave);
-  using E = MfmaEngine<G, D, TS>;
+  using E = MfmaEngine<G, D, PAGES>;
   if (kind == kLaunchListed)
     hipLaunchKernelGGL((listed_decode_kernel<G, E, kWavesPerWg>), grid, block, 0, st, a);
   else if (kind == kLaunchVerified)
@@ -1585,32 +1606,23 @@ void launch_decode_gdt(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st)
                        st, a);
 }
 
-// 16-token pages run engines with the tile shift compiled in (0).
-template <int G, int D>
-void launch_decode_gd(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
-  if (a.ts == 0 && a.tl == 4)
-    launch_decode_gdt<G, D, 0>(a, kind, grid, st);
-  else
-    launch_decode_gdt<G, D, -1>(a, kind, grid, st);
-}
-
-template <int G>
-void launch_decode_g(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
+template <int G, int PAGES>
+void launch_decode_gp(const DecodeArgs &a, int kind, dim3 grid, hipStream_t st) {
   if (a.D == 32)
-    launch_decode_gd<G, 32>(a, kind, grid, st);
+    launch_decode_gdp<G, 32, PAGES>(a, kind, grid, st);
   else if (a.D == 64)
-    launch_decode_gd<G, 64>(a, kind, grid, st);
+    launch_decode_gdp<G, 64, PAGES>(a, kind, grid, st);
   else if (a.D == 256)
-    launch_decode_gd<G, 256>(a, kind, grid, st);
+    launch_decode_gdp<G, 256, PAGES>(a, kind, grid, st);
   else
-    launch_decode_gd<G, 128>(a, kind, grid, st);
+    launch_decode_gdp<G, 128, PAGES>(a, kind, grid, st);
 }
 
 // The reuse step's listed decode with the token append (D = 128, 16-token
 // pages).
 template <int G>
 void launch_append_g(const DecodeArgs &a, const AppendArgs &app, dim3 grid, hipStream_t st) {
-  hipLaunchKernelGGL((listed_append_kernel<G, MfmaEngine<G, 128, 0>, kWavesPerWg>), grid,
+  hipLaunchKernelGGL((listed_append_kernel<G, MfmaEngine<G, 128, kPages16>, kWavesPerWg>), grid,
                      dim3(kWavesPerWg * kWave), 0, st, a, app);
 }
 
@@ -1618,22 +1630,31 @@ void launch_append_g(const DecodeArgs &a, const AppendArgs &app, dim3 grid, hipS
 template <int G>
 void launch_spec_g(const DecodeArgs &a, const ScoreArgs &s, int score_gx, dim3 grid,
                    hipStream_t st) {
-  if (a.ts == 0 && a.tl == 4)
-    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, 0>, kWavesPerWg>), grid,
+  if (a.ts == 0)
+    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, kPages16>, kWavesPerWg>), grid,
                        dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
   else
-    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, -1>, kWavesPerWg>), grid,
+    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, kPagesWide>, kWavesPerWg>), grid,
                        dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
 }
 
 #define CVSA_DECODE_LAUNCHERS(PREFIX, GG)                                                    \
-  PREFIX template void launch_decode_g<GG>(const DecodeArgs &, int, dim3, hipStream_t); \
+  PREFIX template void launch_decode_gp<GG, kPages16>(const DecodeArgs &, int, dim3,          \
+                                                      hipStream_t);                           \
+  PREFIX template void launch_decode_gp<GG, kPagesWide>(const DecodeArgs &, int, dim3,        \
+                                                        hipStream_t);                         \
   PREFIX template void launch_spec_g<GG>(const DecodeArgs &, const ScoreArgs &, int, dim3,   \
                                          hipStream_t);                                         \
   PREFIX template void launch_append_g<GG>(const DecodeArgs &, const AppendArgs &, dim3,      \
                                            hipStream_t);
-#define CVSA_DECODE_EXTERN(GG) CVSA_DECODE_LAUNCHERS(extern, GG)
+#define CVSA_DECODE_EXTERN(GG) \
+  CVSA_DECODE_LAUNCHERS(extern, GG) CVSA_PAGES8_LAUNCHERS(extern, GG)
 #define CVSA_DECODE_INSTANTIATE(GG) CVSA_DECODE_LAUNCHERS(, GG)
+// 8-token pages: decode_pages8_g*.hip.
+#define CVSA_PAGES8_LAUNCHERS(PREFIX, GG)                                             \
+  PREFIX template void launch_decode_gp<GG, kPages8>(const DecodeArgs &, int, dim3,   \
+                                                     hipStream_t);
+#define CVSA_PAGES8_INSTANTIATE(GG) CVSA_PAGES8_LAUNCHERS(, GG)
 
 constexpr int kMaxGroup = 16;       // query heads of one launch: one MFMA tile
 constexpr int kMaxGroupTotal = 128;  // query heads per KV head (launches of 16)

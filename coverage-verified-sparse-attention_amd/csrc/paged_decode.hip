@@ -244,9 +244,14 @@ static int enqueue_decode(const char *name, DecodeArgs a, int G, bool listed,
     a.q_off = off;
     a.work = off == 0 ? work : nullptr;
     switch (min(kMaxGroup, G - off)) {
-#define CVSA_DEC_CASE(GG)                             \
-  case GG:                                            \
-    launch_decode_g<GG>(a, kind, grid, st);    \
+#define CVSA_DEC_CASE(GG)                                       \
+  case GG:                                                      \
+    if (a.tl == 3)                                              \
+      launch_decode_gp<GG, kPages8>(a, kind, grid, st);         \
+    else if (a.ts == 0)                                         \
+      launch_decode_gp<GG, kPages16>(a, kind, grid, st);        \
+    else                                                        \
+      launch_decode_gp<GG, kPagesWide>(a, kind, grid, st);      \
     break;
       CVSA_DEC_CASE(1) CVSA_DEC_CASE(2) CVSA_DEC_CASE(3) CVSA_DEC_CASE(4)
       CVSA_DEC_CASE(5) CVSA_DEC_CASE(6) CVSA_DEC_CASE(7) CVSA_DEC_CASE(8)

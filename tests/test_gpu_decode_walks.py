@@ -77,3 +77,18 @@ def test_walks_across_chunks(gpu, B, H, G, D, bs):
                 assert bool(((o - want[0]).abs() <= 4e-5 * want[3] + 1e-6).all()), (b, h)
                 assert torch.allclose(m, want[1], rtol=0, atol=2e-5), (b, h)
                 assert torch.allclose(l, want[2], rtol=4e-5), (b, h)
+
+
+@pytest.mark.parametrize("B,H,G,D", [(64, 4, 4, 128), (32, 8, 5, 32), (64, 4, 16, 64),
+                                     (64, 4, 2, 256), (128, 2, 1, 128)])
+def test_walks_of_8_token_pages(gpu, B, H, G, D):
+    """The 8-row tiles' engines: more tiles in flight (1 at D = 256, 8 at
+    D = 32) and K and V tiles whose upper half no load writes.  A walk before
+    each one leaves infinities in the LDS that they start from."""
+    shape = (8, 16, H, D)
+    inf = torch.full(shape, float("inf"), device=gpu, dtype=torch.bfloat16)
+    q = torch.ones(B, H * G, D, device=gpu, dtype=torch.bfloat16)
+    bt = torch.zeros(B, 8, device=gpu, dtype=torch.int32)
+    ctx = torch.full((B,), 128, device=gpu, dtype=torch.int32)
+    ops.dense_decode(q, inf, inf, bt, ctx, H, G, 16, return_state=True)
+    test_walks_across_chunks(gpu, B, H, G, D, 8)
