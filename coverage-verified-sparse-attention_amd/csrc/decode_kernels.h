@@ -577,13 +577,17 @@ static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 
 // onto the 8 rows and one tile in flight at D = 128 -> as here, H_kv = 8, G = 4:
 // listed B = 1, 128K 25.0 -> 19.9 us, B = 32 (ragged 8K) 71.0 -> 49.5; dense
 // B = 4, 64K 261.2 -> 186.2.
+// KEYS_AGAIN: other workgroups of the launch read the same keys (a fused check
+// whose scoring part scores the whole cache): K loads leave the lines in the
+// caches.
 enum { kPages16, kPagesWide, kPages8 };
-template <int G, int D, int PAGES>
+template <int G, int D, int PAGES, bool KEYS_AGAIN = false>
 struct MfmaEngine {
   static_assert(G <= 16, "GQA group larger than the MFMA tile");
   static_assert(D == 32 || D == 64 || D == 128 || D == 256, "head dimension");
   static constexpr int kD = D;
   static constexpr int kPages = PAGES;
+  static constexpr bool kKeysOnce = !KEYS_AGAIN;
   // Tiles per page = 1 << tshift(a), rows per tile kRows = 1 << kRowsLog.
   static __device__ __forceinline__ int tshift(const DecodeArgs &a) {
     return PAGES == kPagesWide ? a.ts : 0;
@@ -652,7 +656,7 @@ struct MfmaEngine {
   // The rows of the tile at `base` (wave-uniform) into r.  No tile (live
   // false): nothing is read.  Load i reads rows RPL i + lane / LPR.  The
   // lanes of row `newrow` (-1: none) read nothing.
-  template <bool APP>
+  template <bool APP, bool ONCE>
   __device__ __forceinline__ void fetch(const uint16_t *base, bool live, int newrow,
                                         uint4 (&r)[NL]) const {
     const uint32_t off = voff + (live ? 0u : kRegionSkip);
@@ -660,7 +664,7 @@ struct MfmaEngine {
     for (int i = 0; i < NL; ++i) {
       uint32_t oi = off;
       if (APP && RPL * i + lane / LPR == newrow) oi = kRegionSkip;
-      r[i] = region_load16(base, tile_bytes, oi, RPL * i * row_bytes);
+      r[i] = region_load16<ONCE>(base, tile_bytes, oi, RPL * i * row_bytes);
     }
   }
 
@@ -841,12 +845,12 @@ struct TileChunk {
 // lookup(c) while chunk c - 1 is walked, so the loads run on across chunks.
 // score(lt, ntok, kop) sees each tile's keys first (SCORE).  APP: row new_off
 // of logical tile new_tile is the appended token's (k_new / v_new).
-template <class Engine, bool APP>
+template <class Engine, bool APP, bool ONCE>
 __device__ __forceinline__ void fetch_tile(const DecodeArgs &a, const Engine &eng, int phys,
                                            int lt, int newrow, const uint16_t *cache,
                                            uint4 (&r)[Engine::NL]) {
   const int64_t base = (int64_t)phys * (eng.tile_bytes / 2);
-  eng.template fetch<APP>(cache + base, lt < kUnreadable, newrow, r);
+  eng.template fetch<APP, ONCE>(cache + base, lt < kUnreadable, newrow, r);
 }
 
 template <class Engine, bool APP = false>
@@ -860,9 +864,9 @@ __device__ __forceinline__ void start_walk(const DecodeArgs &a, Engine &eng, con
     // K before V, here and in the walk: the wait for a tile's K then leaves
     // its V in flight.
     __builtin_amdgcn_sched_barrier(0);
-    fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.k_cache, eng.kr[u]);
+    fetch_tile<Engine, APP, Engine::kKeysOnce>(a, eng, phys, lt, newrow, a.k_cache, eng.kr[u]);
     __builtin_amdgcn_sched_barrier(0);
-    fetch_tile<Engine, APP>(a, eng, phys, lt, newrow, a.v_cache, eng.vr[u]);
+    fetch_tile<Engine, APP, true>(a, eng, phys, lt, newrow, a.v_cache, eng.vr[u]);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -898,13 +902,14 @@ __device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int
       const int newrow_n = APP && lt_n == new_tile ? new_off : -1;
       const int ntok = min(1 << tl, max(0, ctx - (lt[u] << tl)));
       eng.template stage_k<APP>(lds, eng.kr[u], newrow, k_new);
-      fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.k_cache, eng.kr[u]);
+      fetch_tile<Engine, APP, Engine::kKeysOnce>(a, eng, phys_n, lt_n, newrow_n, a.k_cache,
+                                                 eng.kr[u]);
       uint4 kop[Engine::NK];
       eng.k_operand(lds, kop);
       if constexpr (SCORE) score(lt[u], ntok, kop);
       const bf16x8_t p = eng.softmax(kop, ntok, lds);
       eng.template stage_v<APP>(lds, eng.vr[u], ntok, newrow, v_new);
-      fetch_tile<Engine, APP>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr[u]);
+      fetch_tile<Engine, APP, true>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr[u]);
       __builtin_amdgcn_sched_barrier(0);
       eng.accumulate(p, lds);
       lt[u] = lt_n;
@@ -1634,8 +1639,13 @@ void launch_spec_g(const DecodeArgs &a, const ScoreArgs &s, int score_gx, dim3 g
     hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, kPages16>, kWavesPerWg>), grid,
                        dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
   else
-    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, kPagesWide>, kWavesPerWg>), grid,
-                       dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
+    // Pages of several tiles: the scoring part reads the selection's keys too.
+    // us a kept check with K loads that stream -> as here (H_kv = 8, G = 4;
+    // before the walk streamed whole K rows): 64-token pages, 128K tokens 62.0 ->
+    // 60.0 (61.4), 512K 221 -> 206 (206), 8 ragged sequences of 32K 108.7 ->
+    // 102.8 (102.7); 32-token pages, 512K 220 -> 207 (207).
+    hipLaunchKernelGGL((score_spec_kernel<G, MfmaEngine<G, 128, kPagesWide, true>, kWavesPerWg>),
+                       grid, dim3(kWavesPerWg * kWave), 0, st, a, s, score_gx);
 }
 
 #define CVSA_DECODE_LAUNCHERS(PREFIX, GG)                                                    \
