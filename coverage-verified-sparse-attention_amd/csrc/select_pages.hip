@@ -38,6 +38,11 @@ namespace cvsa {
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / kWave;
 constexpr int kHistCopies = 16;
+// Histogram copies of a workgroup of NT threads (radix_select): four waves
+// clear and sum 4 of them faster than 16 (8 rows, us a select + gate whose k-th
+// bucket holds more than 64 scores, 16 / 8 / 4 copies: 512 pages 9.6 / 8.7 / 8.2,
+// 1000 pages 11.2 / 9.9 / 9.4).
+constexpr int hist_copies(int NT) { return NT >= kSelThreads ? kHistCopies : 4; }
 constexpr int kHistStride = 257;
 constexpr int kBuckets = 4096;                          // value buckets of the first step
 constexpr int kBucketsPerThread = kBuckets / kSelThreads;
@@ -221,7 +226,7 @@ __device__ __forceinline__ void block_sum2(float &a, float &b, float (*red)[2]) 
   }
 }
 
-// One pass of the MSB radix select: hist_c holds kHistCopies copies of the
+// One pass of the MSB radix select: hist_c holds hist_copies(NT) copies of the
 // histogram of the pass's 8-bit digit over the keys still in the running
 // (behind an LDS barrier); returns the digit holding the krem-th largest of
 // them and krem minus the number of those keys with a higher digit.  Ends
@@ -234,7 +239,7 @@ __device__ __forceinline__ void radix_digit(const uint32_t *hist_c, uint32_t *hi
   for (int i = t; i < 256; i += NT) {
     uint32_t c = 0;
 #pragma unroll
-    for (int j = 0; j < kHistCopies; ++j) c += hist_c[j * kHistStride + i];
+    for (int j = 0; j < hist_copies(NT); ++j) c += hist_c[j * kHistStride + i];
     hist[i] = c;
   }
   lds_barrier();
@@ -269,7 +274,7 @@ __device__ __forceinline__ void radix_digit(const uint32_t *hist_c, uint32_t *hi
 // 4-pass, 8-bit MSB radix select of the k-th largest key among the keys
 // with alive(r) set: returns that key T and k - #(alive keys > T), the
 // number of keys equal to T that the selection takes.  Every lane adds
-// into copy (lane % kHistCopies) of the histogram, rows padded by one word so
+// into copy (lane % hist_copies) of the histogram, rows padded by one word so
 // that the copies of a bin sit in different LDS banks: scores cluster in a
 // few leading digits, so lanes of one instruction often hit the same bin.
 template <int R, int NT, typename Alive>
@@ -283,9 +288,9 @@ __device__ __forceinline__ void radix_select(const float (&val)[R], Alive alive,
 #pragma unroll 1
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
-    for (int i = t; i < kHistCopies * kHistStride; i += NT) hist_c[i] = 0;
+    for (int i = t; i < hist_copies(NT) * kHistStride; i += NT) hist_c[i] = 0;
     lds_barrier();
-    uint32_t *my_hist = hist_c + (lane % kHistCopies) * kHistStride;
+    uint32_t *my_hist = hist_c + (lane % hist_copies(NT)) * kHistStride;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const uint32_t key = order_key(val[r]);
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(NT) void select_topk_kernel(
   constexpr int kWaves = NT / kWave;
   constexpr int NB = kBucketsPerThread * NT;  // value buckets
   __shared__ uint32_t hist[256];
-  __shared__ uint32_t hist_c[kHistCopies * kHistStride];
+  __shared__ uint32_t hist_c[hist_copies(NT) * kHistStride];
   __shared__ uint32_t hist_b[NB];
   __shared__ uint32_t s_cand[kRankCands];
   __shared__ uint32_t wsum[kWaves];
