@@ -769,10 +769,16 @@ __global__ __launch_bounds__(NT) void select_topk_kernel(
           if (t < kWave) {
             const uint32_t mine = t < (int)nb ? s_cand[t] : 0u;
             uint32_t gt = 0, eq = 0;
-            for (uint32_t j = 0; j < nb; ++j) {  // nb is the same in every lane
-              const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j);
-              gt += o > mine;
-              eq += o == mine;
+            // nb is the same in every lane; lanes from nb on hold 0, which no
+            // finite score's key equals or lies below.  Eight lane reads a turn:
+            // one a turn took 1.2 us more at 63 candidates.
+            for (uint32_t j = 0; j < nb; j += 8) {
+#pragma unroll
+              for (uint32_t u = 0; u < 8; ++u) {
+                const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)(j + u));
+                gt += o > mine;
+                eq += o == mine;
+              }
             }
             if (t < (int)nb && gt < kb && kb <= gt + eq) {
               s_T = mine;
