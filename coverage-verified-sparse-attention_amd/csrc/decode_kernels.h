@@ -525,6 +525,7 @@ __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBu
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef short short8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 // RNE bf16 pair (v_cvt_pk_bf16_f32): the bits of f32_to_bf16_bits.
@@ -545,12 +546,15 @@ static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 
 //   S = K Q^T: v_mfma_f32_16x16x32_bf16, four d-chunks of 32.  A operand =
 //     K rows (lane l: token l%16, d 32kk + 8(l/16) .. +8), B operand = Q^T
 //     (loaded once), result lane l: head l%16, tokens 4(l/16) .. +4.
-//   O += P V: P is split into a bf16 high part and a bf16 remainder to keep
-//     ~16 mantissa bits; lane l holds both for head l%16, tokens 4(l/16) ..
-//     +4 (the S result layout), which are the eight A operands of one
-//     v_mfma_f32_16x16x32_bf16 against the tile's V columns taken twice, one
-//     MFMA per 16 columns of d.  The B operand wants 4 tokens of one d column
-//     per lane: ds_read_b64_tr_b16 transposes it out of the row-major V tile.
+//   O += P V: v_mfma_f32_16x16x16_bf16, one 16-column block of d at a time.
+//     The S result layout is the A operand layout of P (head l%16, tokens
+//     4(l/16) .. +4); P is split into a bf16 high part and a bf16 remainder
+//     to keep ~16 mantissa bits, and the two products are added in that
+//     order.  (Both as the eight A operands of one v_mfma_f32_16x16x32_bf16,
+//     V taken twice, round the sum differently and save no time: 17.17 us
+//     listed at 128K, 43.2 at B = 32, 172.1 dense at B = 4, 64K either way.)
+//     The B operand wants 4 tokens of one d column per lane:
+//     ds_read_b64_tr_b16 transposes it out of the row-major V tile.
 //     Result lane l: heads 4(l/16) .. +4, d column 16 blk + l%16.
 // Softmax state: m and the running l of head l%16 live in the four lanes of
 // that head; a rescale of O rows goes through LDS (16 factors per wave).
@@ -748,7 +752,7 @@ struct MfmaEngine {
 
   // Scores of the tile and the softmax state: returns P (head c16, tokens
   // t0 .. t0+3) as bf16 high parts and bf16 remainders.
-  __device__ __forceinline__ bf16x8_t softmax(const uint4 (&kop)[NK], int ntok, Lds &lds) {
+  __device__ __forceinline__ short8_t softmax(const uint4 (&kop)[NK], int ntok, Lds &lds) {
     const int t0 = 4 * (lane >> 4);
     float4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -793,11 +797,13 @@ struct MfmaEngine {
     w.y = cvt_bf16x2(p[2], p[3]);
     w.z = cvt_bf16x2(p[0] - bf16_lo(w.x), p[1] - bf16_hi(w.x));
     w.w = cvt_bf16x2(p[2] - bf16_lo(w.y), p[3] - bf16_hi(w.y));
-    return __builtin_bit_cast(bf16x8_t, w);
+    return __builtin_bit_cast(short8_t, w);
   }
 
-  __device__ __forceinline__ void accumulate(bf16x8_t p, Lds &lds) {
+  __device__ __forceinline__ void accumulate(short8_t p, Lds &lds) {
     const int c16 = lane & 15, t0 = 4 * (lane >> 4);
+    const short4_t high = __builtin_shufflevector(p, p, 0, 1, 2, 3);
+    const short4_t rest = __builtin_shufflevector(p, p, 4, 5, 6, 7);
     typedef __attribute__((address_space(3))) short4_t lds_short4;
     // Lane (c16, grp) names row t0 + c16/4, columns 4 (c16 % 4) .. +4 of a
     // block's 4 x 16 tokens x columns; the transposing read returns it the
@@ -807,9 +813,8 @@ struct MfmaEngine {
     for (int blk = 0; blk < NB; ++blk) {
       const short4_t vb =
           __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(src + 16 * blk));
-      const bf16x8_t vv = __builtin_bit_cast(
-          bf16x8_t, __builtin_shufflevector(vb, vb, 0, 1, 2, 3, 4, 5, 6, 7));
-      o[blk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, vv, o[blk], 0, 0, 0);
+      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(high, vb, o[blk], 0, 0, 0);
+      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(rest, vb, o[blk], 0, 0, 0);
     }
   }
 
@@ -907,7 +912,7 @@ __device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int
       uint4 kop[Engine::NK];
       eng.k_operand(lds, kop);
       if constexpr (SCORE) score(lt[u], ntok, kop);
-      const bf16x8_t p = eng.softmax(kop, ntok, lds);
+      const short8_t p = eng.softmax(kop, ntok, lds);
       eng.template stage_v<APP>(lds, eng.vr[u], ntok, newrow, v_new);
       fetch_tile<Engine, APP, true>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr[u]);
       __builtin_amdgcn_sched_barrier(0);
