@@ -8,6 +8,8 @@ import pytest
 import torch
 
 from cvsa import ops
+from cvsa.ops import _lib
+from cvsa.synthetic import jitter_query, make_paged_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +94,68 @@ def test_walks_of_8_token_pages(gpu, B, H, G, D):
     ctx = torch.full((B,), 128, device=gpu, dtype=torch.int32)
     ops.dense_decode(q, inf, inf, bt, ctx, H, G, 16, return_state=True)
     test_walks_across_chunks(gpu, B, H, G, D, 8)
+
+
+def _whole_head_batch(gpu, ctx, G, max_pages):
+    """256 heads of up to 301 pages: one workgroup walks a head, 76 tiles a wave."""
+    return make_paged_inputs(32, 8 * G, 8, 128, ctx, seed=5, device=gpu, max_pages=max_pages,
+                             spare_blocks=64)
+
+
+def test_folded_append_across_chunks(gpu):
+    """The appended token's page at the edges of a wave's chunks (tiles 0, 63,
+    64 and the last of waves 0 and 3), mid-page and on a page that the append
+    allocates: bit for bit the append followed by the listed decode."""
+    B, H, G, last = 32, 8, 4, 300
+    ctx = [16 * last + (0, 5, 15)[b % 3] for b in range(B)]
+    inp = _whole_head_batch(gpu, ctx, G, last + 1)
+    alloc = torch.tensor([-(-c // 16) for c in ctx], dtype=torch.int32, device=gpu)
+    g = torch.Generator().manual_seed(9)
+    pi = torch.zeros(B, H, last + 1, dtype=torch.int32)
+    nph = torch.zeros(B, H, dtype=torch.int32)
+    places = (0, 3, 252, 255, 256, 259, -1, None)  # entry that lists the new page
+    for b in range(B):
+        for h in range(H):
+            at, n = places[(b + h) % 8], last + 1 - (b + 3 * h) % 4
+            pages = torch.randperm(last, generator=g)[:n - (at is not None)].tolist()
+            if at is not None:
+                pages.insert(len(pages) if at < 0 else at, last)
+            pi[b, h, :len(pages)] = torch.tensor(pages)
+            nph[b, h] = len(pages)
+    pi, nph = pi.to(gpu), nph.to(gpu)
+    kn, vn = (torch.randn(B, H, 128, generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    slots, fresh = [], inp.used_blocks
+    for c in ctx:
+        slots += [c, fresh if c % 16 == 0 else -1]
+        fresh += c % 16 == 0
+    state = [inp.k_cache.clone(), inp.v_cache.clone(), inp.block_tables.clone(),
+             inp.context_lens.clone(), alloc.clone()]
+    out = ops.sparse_decode_append(inp.q, *state[:4], pi, nph, kn, vn, state[4], slots, H, G, 16)
+    ref = [inp.k_cache, inp.v_cache, inp.block_tables, inp.context_lens, alloc]
+    ops.append_kv(kn, vn, *ref, 0, inp.used_blocks, 16)
+    want = ops.sparse_decode(inp.q, ref[0], ref[1], ref[2], pi, nph, ref[3], H, G, 16)
+    assert torch.equal(out, want)
+    assert all(torch.equal(a, b) for a, b in zip(state, ref))
+
+
+@pytest.mark.parametrize("predict,tau", [(1, 0.0), (2, 1.5)])
+def test_walk_scores_across_chunks(gpu, predict, tau):
+    """Page scores written by the walks of a fused check (the kept selection's
+    and the dense one) whose waves run over several chunks: bit for bit the
+    page scoring's, and the check that of a plan without speculation."""
+    H, G, budget = 8, 2, 290
+    ctx = [16 * 300 - (b * 7) % 40 for b in range(32)]
+    inp = _whole_head_batch(gpu, ctx, G, 300)
+    ctx, bt = inp.context_lens, inp.block_tables
+    ps = ops.score_pages(inp.q, inp.k_cache, bt, ctx, H, G, 16)
+    sel, nph = ops.select_topk(ps, budget, ctx, 16)
+    q = jitter_query(inp.q, 0.5, 3)
+    plans = [ops.StepPlan(inp.q, inp.k_cache, inp.v_cache, bt, ctx, H, G, 16, budget, tau,
+                          sel.clone(), nph.clone(), speculate=s) for s in (True, False)]
+    plans[0].spec_state[0] = predict
+    got, want = (p.run(_lib.STEP_LAZY_CHECK, q) for p in plans)
+    assert plans[0].spec_state.tolist() == [predict, predict]
+    assert torch.equal(plans[0].page_scores, ops.score_pages(q, inp.k_cache, bt, ctx, H, G, 16))
+    assert torch.equal(got, want)
+    assert torch.equal(plans[0].accept, plans[1].accept)
+    assert torch.equal(plans[0].page_indices, plans[1].page_indices)
