@@ -37,8 +37,8 @@
 // increment, an agent-scope acquire fence in the last arriver): the same
 // bits, but the L2 writeback and invalidate those fences compile to cost
 // the cfg3 listed decode 31.5 us against 19.3 us (one rejected head 67 vs
-// 37 us, dense 135 vs 96 us), so the default build keeps the cache-policy
-// protocol.
+// 37 us, dense 135 vs 96 us; measured with an engine that took 19.3 us where
+// this one takes 17.1), so the default build keeps the cache-policy protocol.
 //
 // Head modes: a listed head walks page_indices[b,h,:n_per_head]; an
 // all-pages head walks pages 0..n_valid-1 (dense decode).  In verified mode
@@ -70,7 +70,7 @@ constexpr int kMaxSplits = 256;            // partials per head (and workgroups 
 // Waves per workgroup, one per SIMD.  Eight waves (two per SIMD, the same
 // tiles in flight per wave) measured slower: the listed decode 17.3 against
 // 17.1 us at cfg3 and 44.4 against 43.2 us at B = 32 (ragged 8K contexts),
-// dense at B = 4, 64K 186 against 178 us.
+// dense at B = 4, 64K 186 against 178 us (172 since the chunks run on).
 constexpr int kWavesPerWg = 4;
 constexpr int kMinPagesPerWave = 2;        // pages per wave of a split, at least
 
@@ -520,8 +520,7 @@ __device__ __forceinline__ void merge_partials(const DecodeArgs &a, const PartBu
 // tiles (one from D = 128 on) are in registers at a time: each tile is staged
 // to LDS as soon as it arrives and the loads of the tile PD further on are
 // issued into the same registers at once, so a wave always has about PD tiles
-// in flight; finish() leaves the wave's (o, m, l)
-// in LDS.
+// in flight; finish() leaves the wave's (o, m, l) in LDS.
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
@@ -571,8 +570,10 @@ static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 
 // range and are dropped there (prefetches that read a wave's last tile again
 // instead cost the cfg3 listed decode a quarter more requests).  With the
 // engine of two tiles in flight the kernels took: listed 19.1 -> 17.1 us at
-// cfg3, 47.2 -> 43.2 us at B = 32 (ragged 8K), 10.3 -> 9.0 us at B = 1, 8K;
-// dense at B = 4, 64K, G = 8 185-191 -> 178 us.
+// cfg3, 47.2 -> 43.2 us at B = 32 (ragged 8K), 10.3 -> 8.9 us at B = 1, 8K;
+// dense at B = 4, 64K, G = 8 185 -> 172 us.  Launches of fewer workgroups than
+// CUs gain as well (136 / 192 / 248 heads, 8K, a workgroup each: 34.6 -> 31.1,
+// 37.5 -> 35.3, 47.0 -> 43.5 us).
 //
 // PAGES: kPages16 (one 16-row tile per page), kPagesWide (2^ts of them) or
 // kPages8.  An 8-token page is a tile of 8 rows: rows 8 .. 15 of the two LDS
@@ -845,19 +846,16 @@ struct TileChunk {
   int phys = 0, lt = kNoTile;
 };
 
-// One wave's walk over npw tiles.  `cur` is the first chunk's tiles, whose
-// first PD tiles' loads are in flight (start_walk); chunk c's tiles come from
-// lookup(c) while chunk c - 1 is walked, so the loads run on across chunks.
-// score(lt, ntok, kop) sees each tile's keys first (SCORE).  APP: row new_off
-// of logical tile new_tile is the appended token's (k_new / v_new).
+// The rows of physical tile phys into r; logical tile lt from kUnreadable on:
+// nothing is read.
 template <class Engine, bool APP, bool ONCE>
-__device__ __forceinline__ void fetch_tile(const DecodeArgs &a, const Engine &eng, int phys,
-                                           int lt, int newrow, const uint16_t *cache,
-                                           uint4 (&r)[Engine::NL]) {
+__device__ __forceinline__ void fetch_tile(const Engine &eng, int phys, int lt, int newrow,
+                                           const uint16_t *cache, uint4 (&r)[Engine::NL]) {
   const int64_t base = (int64_t)phys * (eng.tile_bytes / 2);
   eng.template fetch<APP, ONCE>(cache + base, lt < kUnreadable, newrow, r);
 }
 
+// Requests the first PD tiles of a walk (those of the first chunk, `cur`).
 template <class Engine, bool APP = false>
 __device__ __forceinline__ void start_walk(const DecodeArgs &a, Engine &eng, const TileChunk &cur,
                                            int new_tile = -1, int new_off = -1) {
@@ -869,13 +867,18 @@ __device__ __forceinline__ void start_walk(const DecodeArgs &a, Engine &eng, con
     // K before V, here and in the walk: the wait for a tile's K then leaves
     // its V in flight.
     __builtin_amdgcn_sched_barrier(0);
-    fetch_tile<Engine, APP, Engine::kKeysOnce>(a, eng, phys, lt, newrow, a.k_cache, eng.kr[u]);
+    fetch_tile<Engine, APP, Engine::kKeysOnce>(eng, phys, lt, newrow, a.k_cache, eng.kr[u]);
     __builtin_amdgcn_sched_barrier(0);
-    fetch_tile<Engine, APP, true>(a, eng, phys, lt, newrow, a.v_cache, eng.vr[u]);
+    fetch_tile<Engine, APP, true>(eng, phys, lt, newrow, a.v_cache, eng.vr[u]);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
+// One wave's walk over npw tiles.  `cur` is the first chunk's tiles, whose
+// first PD tiles' loads are in flight (start_walk); chunk c's tiles come from
+// lookup(c) while chunk c - 1 is walked, so the loads run on across chunks.
+// score(lt, ntok, kop) sees each tile's keys first (SCORE).  APP: row new_off
+// of logical tile new_tile is the appended token's (k_new / v_new).
 template <class Engine, bool APP, bool SCORE, class Lookup, class Score>
 __device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int npw, int ctx,
                                            TileChunk cur, Lookup lookup, Score score,
@@ -907,14 +910,14 @@ __device__ __forceinline__ void walk_tiles(const DecodeArgs &a, Engine &eng, int
       const int newrow_n = APP && lt_n == new_tile ? new_off : -1;
       const int ntok = min(1 << tl, max(0, ctx - (lt[u] << tl)));
       eng.template stage_k<APP>(lds, eng.kr[u], newrow, k_new);
-      fetch_tile<Engine, APP, Engine::kKeysOnce>(a, eng, phys_n, lt_n, newrow_n, a.k_cache,
+      fetch_tile<Engine, APP, Engine::kKeysOnce>(eng, phys_n, lt_n, newrow_n, a.k_cache,
                                                  eng.kr[u]);
       uint4 kop[Engine::NK];
       eng.k_operand(lds, kop);
       if constexpr (SCORE) score(lt[u], ntok, kop);
       const short8_t p = eng.softmax(kop, ntok, lds);
       eng.template stage_v<APP>(lds, eng.vr[u], ntok, newrow, v_new);
-      fetch_tile<Engine, APP, true>(a, eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr[u]);
+      fetch_tile<Engine, APP, true>(eng, phys_n, lt_n, newrow_n, a.v_cache, eng.vr[u]);
       __builtin_amdgcn_sched_barrier(0);
       eng.accumulate(p, lds);
       lt[u] = lt_n;
@@ -1130,8 +1133,9 @@ __device__ __forceinline__ int listed_pps(const DecodeArgs &a, int n, int ts) {
 // outputs).  Partial row of (split, head) = head * n_splits + split.
 // With APP, the walk's sequence appends token nt in this launch: the
 // context length is nt's page * 16 + row + 1 (16-token pages), and nt's page
-// reads that row from nt's rows (Engine::fetch_new) and, when the append
-// allocates the page, its block from nt.
+// takes that row from nt's rows (its loads are dropped, stage_k and stage_v
+// put the new row in place) and, when the append allocates the page, its
+// block from nt.
 // With SCORE and a.spec_scores, the walk also writes the page score of
 // every page it walks (Engine::page_score; qrep: this wave's LDS copy of the
 // 16 q_rep segments, 16-token pages).
