@@ -577,10 +577,10 @@ static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 
 //
 // PAGES: kPages16 (one 16-row tile per page), kPagesWide (2^ts of them) or
 // kPages8.  An 8-token page is a tile of 8 rows: rows 8 .. 15 of the two LDS
-// tiles are no token's (K: never looked at, V: zeros), are not read from
-// memory, and twice as many tiles are in flight.  With 16-row loads folded
-// onto the 8 rows and one tile in flight at D = 128 -> as here, H_kv = 8, G = 4:
-// listed B = 1, 128K 25.0 -> 19.9 us, B = 32 (ragged 8K) 71.0 -> 49.5; dense
+// tiles are no token's (K: their scores are masked, V: zeros), nothing is read
+// from memory for them, and twice as many tiles are in flight.  With 16-row
+// loads folded onto the 8 rows and one tile in flight at D = 128 -> as here,
+// H_kv = 8, G = 4: listed B = 1, 128K 25.0 -> 19.9 us, B = 32 (ragged 8K) 71.0 -> 49.5; dense
 // B = 4, 64K 261.2 -> 186.2.
 // KEYS_AGAIN: other workgroups of the launch read the same keys (a fused check
 // whose scoring part scores the whole cache): K loads leave the lines in the

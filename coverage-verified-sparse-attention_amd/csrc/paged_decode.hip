@@ -35,19 +35,18 @@ __global__ void fill_zero_kernel(uint32_t *p, size_t n_words) {
 
 
 // Launch plan.  Listed launches (every head walks its page list) use the
-// static split grid of listed_decode_kernel: ~target_workgroups()
-// workgroups spread over the heads, at least kMinPagesPerWg pages per split,
-// at most kMaxSplits splits per head.  Verified and dense launches use the
-// stream-K grid of streamk_decode_kernel: kTargetWorkgroups, fewer when
-// even the largest possible page list (every head walking all W pages) would
-// give a workgroup less than min_sk_tiles one-tile pages, or less than
-// kMinPagesPerWg pages of several tiles (2^ts of them: 16 to 64 tiles); the
-// kernel narrows it to the tiles actually walked.  Pages of several tiles do
-// not get one workgroup per min_sk_tiles tiles: callers size the
-// workspace without the block size, for a workgroup per kMinPagesPerWg pages.
-// (One per 16 such pages took a dense 8K call, H_kv = 8, from
-// 16.3 to 23.1 us with 64-token pages and from 23.2 to 36.8 with 128-token
-// ones.)
+// static split grid of listed_decode_kernel: ~kTargetWorkgroups workgroups
+// spread over the heads, at least kMinPagesPerWg pages per split, at most
+// kMaxSplits splits per head.  Verified and dense launches use the stream-K
+// grid of streamk_decode_kernel: kTargetWorkgroups, fewer when even the
+// largest possible page list (every head walking all W pages) would give a
+// workgroup less than min_sk_tiles one-tile pages, or less than kMinPagesPerWg
+// pages of several tiles (2^ts each: 16 to 64 tiles); the kernel narrows it to
+// the tiles actually walked.  Pages of several tiles do not get a workgroup per
+// min_sk_tiles tiles because callers size the workspace without the block
+// size, for a workgroup per kMinPagesPerWg pages.  (One per 16 such pages took
+// a dense 8K call, H_kv = 8, from 16.3 to 23.1 us with 64-token pages and from
+// 23.2 to 36.8 with 128-token ones.)
 struct DecodeLaunch {
   bool streamk;
   int grid_x, grid_y;
