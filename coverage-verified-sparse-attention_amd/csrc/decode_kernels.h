@@ -550,8 +550,9 @@ static_assert(((int64_t)kMaxPagesWide << 3) <= kNoTile - kUnreadable, "pages of 
 //     4(l/16) .. +4); P is split into a bf16 high part and a bf16 remainder
 //     to keep ~16 mantissa bits, and the two products are added in that
 //     order.  (Both as the eight A operands of one v_mfma_f32_16x16x32_bf16,
-//     V taken twice, round the sum differently and save no time: 17.17 us
-//     listed at 128K, 43.2 at B = 32, 172.1 dense at B = 4, 64K either way.)
+//     V taken twice, round the sum differently and save no time: 17.1 us
+//     listed at 128K, 43.2 at B = 32, 172.1 dense at B = 4, 64K either way,
+//     26.1 against 25.6 a scoring step at B = 1, 8K.)
 //     The B operand wants 4 tokens of one d column per lane:
 //     ds_read_b64_tr_b16 transposes it out of the row-major V tile.
 //     Result lane l: heads 4(l/16) .. +4, d column 16 blk + l%16.
@@ -810,13 +811,18 @@ struct MfmaEngine {
     // block's 4 x 16 tokens x columns; the transposing read returns it the
     // four tokens t0 .. t0+3 of column c16.
     const uint16_t *src = &lds.t.v[(t0 + (c16 >> 2)) * kRow + 4 * (c16 & 3)];
+    // The second product of a block depends on the first: one pass per part
+    // over the blocks leaves no wait between them (scoring step at B = 1, 8K
+    // 26.3 -> 25.6 us, dense B = 1, 8K 14.30 -> 14.09, 32K 28.2 -> 27.9).
+    short4_t vb[NB];
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk) {
-      const short4_t vb =
-          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(src + 16 * blk));
-      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(high, vb, o[blk], 0, 0, 0);
-      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(rest, vb, o[blk], 0, 0, 0);
+      vb[blk] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(src + 16 * blk));
+      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(high, vb[blk], o[blk], 0, 0, 0);
     }
+#pragma unroll
+    for (int blk = 0; blk < NB; ++blk)
+      o[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(rest, vb[blk], o[blk], 0, 0, 0);
   }
 
   __device__ __forceinline__ void finish(Lds &lds, float *s_m, float *s_l) {
