@@ -1330,12 +1330,13 @@ constexpr int kSpecHeadPPW = 16;
 // kernel, rewrites.
 // One launch lets the decode's dependent metadata loads and split hand-off
 // overlap the scoring stream without a second stream and its events.
-// Up to four waves per SIMD (128 registers; groups above 8 would spill there
-// and take 168): the decode and scoring workgroups of a cfg3 launch all run
-// at once.  Reading the kept selection's keys once: kept check 64.0 -> 61.1 us
+// Three waves per SIMD: the decode and scoring workgroups of a cfg3 launch all
+// run at once.  Held to four (128 of the 137 registers it takes at G <= 8) a
+// kept check takes 18.9 instead of 18.2 us at 8K, 60.2 instead of 59.8 at 128K,
+// 116.7 instead of 114.4 at B = 8, 32K.  Reading the kept selection's keys once: kept check 64.0 -> 61.1 us
 // at cfg3 (16 pages per scoring wave; 8 and 32 measured 61.2 and 62.0).
 template <int G, class Engine, int NW>
-__global__ __launch_bounds__(NW * kWave, Engine::kPages != kPages16 ? 2 : G > 8 ? 3 : 4)
+__global__ __launch_bounds__(NW * kWave, Engine::kPages != kPages16 ? 2 : 3)
 void score_spec_kernel(const DecodeArgs a, const ScoreArgs s, int score_gx) {
   __shared__ WalkLds<G, Engine, NW> L;
   __shared__ uint4 s_qrep[NW][16];  // decode part: q_rep per wave
